@@ -122,6 +122,10 @@ struct DevSub {
 };
 
 constexpr size_t kGidxMaxBytes = 24 * 1024;
+// hubs above this degree get all 16 wavefronts of a workgroup in k_hub_seq: a
+// list of 4096 entries takes 4 wavefronts some 50 us, as long as a gathering
+// step's other launch takes on the smallest graphs with such hubs
+constexpr int64_t kHubBigDegree = 4096;
 
 }  // namespace
 
@@ -181,6 +185,7 @@ struct pg_ctx {
     int64_t built_deg = -1, built_chunk = -1, built_high = -1, built_mid = -1;
     int32_t n_hub = 0, hi_end = 0, mid_end = 0;  // [0,n_hub) hubs, [n_hub,hi_end) high, [hi_end,mid_end) mid
     int32_t n_hub_items = 0, n_slots = 0;
+    int32_t n_big = 0;  // leading hubs above kHubBigDegree: k_hub_seq gives them a whole workgroup
     DevBuf d_hub_items, d_slot_begin;
     DevBuf d_hub_iota;  // [n_hub+1] h -> h: one partial row per hub (column-split hub launches)
     // per-call workspace
@@ -285,6 +290,8 @@ int build_buckets(pg_ctx* c)
     }
     slot_begin[nh] = (int32_t)items.size();
     c->n_hub = nh;
+    c->n_big = 0;
+    while (c->n_big < nh && deg(c->n_big) > kHubBigDegree) ++c->n_big;
     c->hi_end = hi;
     c->mid_end = mid;
     c->n_hub_items = (int32_t)items.size();
@@ -500,7 +507,7 @@ size_t sub_lds_max_t(const pg_ctx* c, const pg_plan* p, const DevSub& d, int B, 
         // whole rows (RUNS_SEQ, LDS independent of B) or by teams of
         // max(8, cl) lanes, one group
         const int cl = std::max(8, cl_of(aux, B, p->k, d.Wy, d.Wa, rc));
-        m = std::max(m, hub_seq_lds_bytes(p->K));
+        m = std::max(m, hub_seq_lds_bytes(p->k));
         if (d.xidx_g.p && runs_seq_for(c, d.Wa, runs_used_per_mille(p, d, AUX_GATHER))) {
             SubArgs<T> a{};
             a.B = B;
@@ -835,8 +842,8 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
 // column order, starting from zero), so the FP32 sums are the reference's,
 // bit for bit:
 //  - hubs: one partial row per hub, each value one running sum over the whole
-//    neighbour list, by k_hub_seq (a wavefront per 64 values with 32-56 row
-//    loads in flight per lane);
+//    neighbour list, by k_hub_seq (the wavefronts of a workgroup share the
+//    list and hand the running sums on);
 //  - the other vertices: a team with the whole neighbour list, one
 //    neighbour group, by whole rows (RUNS_SEQ, when `rows`) or by gathers;
 //  - the finishing launch adds each hub's single partial row to zero and
@@ -870,7 +877,7 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         h.item_base = 0;
         h.n_items = c->n_hub;
         record(c, sizeof(T) == 4 ? "k_hub_seq<float>" : "k_hub_seq<double>", share(c->h_rowptr[c->n_hub], 0), true);
-        HIP_TRY(c, launch_hub_seq<T>(h, cus, c->blocks_per_cu, hs));
+        HIP_TRY(c, launch_hub_seq<T>(h, c->n_big, hs));
         record(c, "", 0, false);
         return PG_OK;
     };
