@@ -181,6 +181,7 @@ struct pg_ctx {
     bool has_transpose = false, symmetric = false;
     DevBuf d_erow, d_tr, d_wT32, d_wT64, d_grad, d_grad_out;
     DevBuf d_rowptr, d_col, d_ent, d_perm, d_w32, d_w64, d_wsrc;
+    bool w64_filled = false;  // d_w64 holds the current weights (widened from d_w32 for the first FP64 pass)
     // degree buckets and hub work items for the current options
     int64_t built_deg = -1, built_chunk = -1, built_high = -1, built_mid = -1;
     int32_t n_hub = 0, hi_end = 0, mid_end = 0;  // [0,n_hub) hubs, [n_hub,hi_end) high, [hi_end,mid_end) mid
@@ -931,6 +932,18 @@ struct PassBufs {
     double* tmp;
 };
 
+// The entry weights of FP64 passes: the FP32 ones widened, by the first such
+// pass after they were set (a streaming pass, where a second gather from the
+// caller's order costs what the first did).  FP32 passes need none of it.
+template <typename T>
+int fill_weights(pg_ctx* c)
+{
+    if (sizeof(T) == 4 || !c->weighted || c->w64_filled) return PG_OK;
+    HIP_TRY(c, launch_widen_weights(c->d_w64.as<double>(), c->d_w32.as<float>(), c->nnz, c->stream));
+    c->w64_filled = true;
+    return PG_OK;
+}
+
 // the device memory a pass's buffers are placed in: the context's arena, or
 // the static scratch during pg_count_noalloc
 char* arena_base(const pg_ctx* c) { return c->arena_override ? c->arena_override : c->d_arena.as<char>(); }
@@ -1391,6 +1404,8 @@ int count_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors, uin
     }
     c->last_tile = tile;
     c->last_recompute = 0;
+    rc = fill_weights<T>(c);
+    if (rc) return rc;
     if (c->autotune) {
         int tuned_tile = tile;
         rc = autotune<T>(c, p, tile, &tuned_tile);
@@ -1496,6 +1511,8 @@ int count_multi_impl(pg_ctx* c, int np, const pg_plan* const* plans, const int32
     *done = false;
     if (!c->use_graphs || c->timing || np < 2) return PG_OK;
     int rc = build_buckets(c);
+    if (rc) return rc;
+    rc = fill_weights<T>(c);
     if (rc) return rc;
     const size_t tsz = sizeof(T);
     const std::vector<int64_t> entry = current_settings(c);
@@ -2101,6 +2118,8 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
     if (rc) return rc;
     if (!c->symmetric)
         return set_err(c, PG_ERR_INVALID, "gradients need a symmetric pattern (every entry's transpose present)");
+    rc = fill_weights<T>(c);
+    if (rc) return rc;
     const size_t tsz = sizeof(T);
     size_t budget;
     if (c->mem_budget_mb > 0) {
@@ -2176,13 +2195,14 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         drop_graphs(c);
         HIP_TRY(c, c->d_arena.alloc(gp.total));
     }
-    if (c->weighted) {
-        HIP_TRY(c, c->d_wT32.alloc(c->nnz * 4));
-        HIP_TRY(c, c->d_wT64.alloc(c->nnz * 8));
-        HIP_TRY(c, launch_gather_weights_f32(c->d_wT32.as<float>(), c->d_w32.as<float>(), c->d_tr.as<int32_t>(),
-                                             c->nnz, c->stream));
-        HIP_TRY(c, launch_gather_weights_f64(c->d_wT64.as<double>(), c->d_w32.as<float>(), c->d_tr.as<int32_t>(),
-                                             c->nnz, c->stream));
+    // the transposed gathers' weights, in the tables' type: read by the steps
+    // whose aux child has a table (a star has none)
+    bool transposed = false;
+    for (auto& d : p->subs) transposed |= d->aa > 1;
+    if (c->weighted && transposed) {
+        DevBuf& wT = tsz == 4 ? c->d_wT32 : c->d_wT64;
+        HIP_TRY(c, wT.alloc(c->nnz * tsz));
+        HIP_TRY(c, launch_gather_weights<T>(wT.as<T>(), c->d_w32.as<float>(), c->d_tr.as<int32_t>(), c->nnz, c->stream));
     }
     HIP_TRY(c, c->d_grad.alloc(std::max<int64_t>(c->nnz, 1) * 8));
     HIP_TRY(c, launch_zero_f64(c->d_grad.as<double>(), c->nnz, c->stream));
@@ -2817,8 +2837,8 @@ extern "C" int pg_graph_set_weights(pg_ctx* c, const float* vals, int on_device)
     }
     HIP_TRY(c, c->d_w32.alloc(std::max<int64_t>(c->nnz, 1) * 4));
     HIP_TRY(c, c->d_w64.alloc(std::max<int64_t>(c->nnz, 1) * 8));
-    HIP_TRY(c, launch_gather_weights_f32(c->d_w32.as<float>(), src, c->d_ent.as<int32_t>(), c->nnz, c->stream));
-    HIP_TRY(c, launch_gather_weights_f64(c->d_w64.as<double>(), src, c->d_ent.as<int32_t>(), c->nnz, c->stream));
+    c->w64_filled = false;
+    HIP_TRY(c, launch_gather_weights<float>(c->d_w32.as<float>(), src, c->d_ent.as<int32_t>(), c->nnz, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     c->weighted = true;
     if (!was_weighted || old32 != c->d_w32.p || old64 != c->d_w64.p) c->generation++;
@@ -3378,6 +3398,8 @@ int count_noalloc_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* col
         }
     } guard(c);
     c->last_tile = tile;
+    const int wrc = fill_weights<T>(c);
+    if (wrc) return wrc;
     double raw[64];
     for (int first = 0; first < ncol; first += tile) {
         const int B = std::min(tile, ncol - first);

@@ -222,8 +222,10 @@ hipError_t launch_edge_colors(uint8_t* ecol, const int32_t* col, const uint8_t* 
 constexpr int kReduceBlocks = 256;
 hipError_t launch_root_reduce(const double* vals, int64_t n, int B, double* tmp, double* out, hipStream_t st);
 // dst[i] = (T) src[ent[i]] (weights into internal entry order)
-hipError_t launch_gather_weights_f32(float* dst, const float* src, const int32_t* ent, int64_t nnz, hipStream_t st);
-hipError_t launch_gather_weights_f64(double* dst, const float* src, const int32_t* ent, int64_t nnz, hipStream_t st);
+template <typename T>
+hipError_t launch_gather_weights(T* dst, const float* src, const int32_t* ent, int64_t nnz, hipStream_t st);
+// dst[i] = (double) src[i]
+hipError_t launch_widen_weights(double* dst, const float* src, int64_t nnz, hipStream_t st);
 
 // ---- adjoint DP -------------------------------------------------------
 // Per vertex and coloring, from G = dR/dT_s (ones at the root), the main row
