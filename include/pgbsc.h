@@ -95,11 +95,12 @@ const char* pg_last_error(const pg_ctx* ctx);
  *                  other vertices' launch (default); 0 = one after the other (same results)
  *   "color_runs"   whole-row neighbour sums: 1 always (rows up to 512 values), 0 never,
  *                  -1 by row width and used share (default)
- *   "fuse_grad"    pg_count_grad with kept tables: 1 = the forward keeps Y of the steps whose
- *                  transposed gather runs by colour runs, and that gather also takes the
+ *   "fuse_grad"    pg_count_grad with kept tables: 1 = the forward keeps the Y that the adjoint
+ *                  reads, and the transposed gather (by colour runs or per lane) also takes the
  *                  entries' gradients (default); 0 = a gradient gather recomputes Y
- *   "fuse_min_width" with fuse_grad: also fuse steps whose dY rows have at least this many
- *                  values, by colour runs whatever share of a row a vertex uses (default 128)
+ *   "fuse_min_width" with fuse_grad: steps whose dY rows have at least this many values, and
+ *                  whose per-lane gather has no index table, fuse by colour runs whatever share
+ *                  of a row a vertex uses (default 128)
  *   "node_fp32"    pg_count_grad with FP32 tables: 1 = the adjoint's split sums in FP32
  *                  (fused multiply-adds, default), 0 = in FP64
  *   "node_rows"    pg_count_grad: 1 = staged node launches over rows of 32+ values take a

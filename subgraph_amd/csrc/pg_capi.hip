@@ -164,7 +164,7 @@ struct pg_ctx {
     int64_t fuse_grad = 1;      // adjoint: forward Y kept and the gradient taken in the transposed gather
     int64_t node_fp32 = 1;      // adjoint node sums of FP32 tables: 1 FP32 fused multiply-adds, 0 FP64
     int64_t runs_g_min = 128;   // gradient gathers by colour runs from this row width (color_runs -1)
-    int64_t fuse_min_width = 128;   // fused gradient also for dY rows of at least this many values
+    int64_t fuse_min_width = 128;   // fused gradient by whole rows also from this many values without an index table
     int64_t seq_max_width = 512;    // exact-order gathers by whole rows (RUNS_SEQ) up to this row width
     int64_t node_rows = 1;      // adjoint node launches: a thread per value over a group's rows (1) or per (row, value)
     int64_t reg_cols = 0;       // values per lane of gathers: 0 one for rows under kRegCols, else 1 or 4
@@ -399,7 +399,8 @@ int aux_mode_for(const pg_ctx* c, const pg_plan* p, const DevSub& d)
 int rc_for(const pg_ctx* c, int aux, int B, int Wy)
 {
     (void)B;
-    const bool gather = aux == AUX_GATHER || aux == AUX_GATHER_G || aux == AUX_GATHER_T;
+    const bool gather =
+        aux == AUX_GATHER || aux == AUX_GATHER_G || aux == AUX_GATHER_T || aux == AUX_GATHER_TG;
     if (!gather) return kRegCols;
     if (c->reg_cols != 0) return (int)c->reg_cols;
     return Wy < kRegCols ? 1 : kRegCols;
@@ -1726,20 +1727,55 @@ size_t table_bytes(const pg_ctx* c, const DevSub& d, int B, size_t tsz)
     return align_up((size_t)c->n_act * B * d.Wo * tsz, 256);
 }
 
-// Whether the adjoint of step d takes its entries' gradients in the
-// transposed gather (RUNS_TG, from the forward's kept Y) instead of a
-// gradient gather that recomputes Y, with option fuse_grad on: when the
-// transposed gather of d runs by colour runs, or its dY rows have at least
-// fuse_min_width values (then by colour runs too, whatever share of a row a
-// vertex uses: one whole-row read per entry replaces the gradient gather's
-// read of the aux rows and the transposed gather's partial one).
+// Whether the adjoint of step d takes its entries' gradients in a transposed
+// gather by whole rows (RUNS_TG, from the forward's kept Y), with option
+// fuse_grad on: when the transposed gather of d runs by colour runs (half or
+// more of a row used), or its dY rows have at least fuse_min_width values and
+// the per-lane gather has no index table for them (without one it does its set
+// arithmetic per value).  With one, the per-lane gather reads only the used
+// part of a row (AUX_GATHER_TG): the 12-vertex tree's 165-value steps, 27%
+// used, R-MAT scale 20, 4 colorings: 9.8 ms a step per lane, 18.5 ms by whole
+// rows.
 bool fused_grad_step(const pg_ctx* c, const pg_plan* p, const DevSub& d)
 {
     if (!c->fuse_grad || d.aa <= 1 || runs_values_per_lane(d.Wy) == 0) return false;
     // its LDS (the G_aux and own rows per team) must fit at either precision
     if (runs_tg_lds_bytes<double>(p->K, d.Wa) > kLdsLimit) return false;
     return runs_mode_for(c, AUX_GATHER_T, d.Wy, runs_used_per_mille(p, d, AUX_GATHER_T)) == RUNS_T ||
-           (c->color_runs != 0 && d.Wy >= c->fuse_min_width);
+           (c->color_runs != 0 && !d.gidxT.p && d.Wy >= c->fuse_min_width);
+}
+
+// Whether the per-lane transposed gather of step d takes its entries'
+// gradients too (AUX_GATHER_TG, option fuse_grad), where fused_grad_step does
+// not apply: one gather of the neighbours' dY rows instead of one of their aux
+// rows and one of their dY rows.  The node launch then needs the forward's Y,
+// unless the main child is a leaf.  R-MAT scale 20, 4 colorings, a 55-value
+// step of the 12-vertex tree: 3.3 ms against 6.5 + 3.1; 7-vertex tree on a
+// uniform graph, FP64, 5 colorings, its three steps: 2.4 ms against 2.6 + 2.3.
+bool lane_grad_step(const pg_ctx* c, const pg_plan* p, const DevSub& d)
+{
+    return c->fuse_grad && d.aa > 1 && !fused_grad_step(c, p, d) &&
+           runs_mode_for(c, AUX_GATHER_T, d.Wy, runs_used_per_mille(p, d, AUX_GATHER_T)) < 0;
+}
+
+// The arguments of step d's transposed gather: G_aux from the neighbours' dY.
+template <typename T>
+SubArgs<T> transposed_args(const pg_ctx* c, const DevSub& d, int B, SubArgs<T> t, const T* dY, T* Ga)
+{
+    t.out_mode = OUT_Y;
+    if (c->weighted) t.w = sizeof(T) == 4 ? (const T*)c->d_wT32.p : (const T*)c->d_wT64.p;
+    t.aux = dY;
+    t.lda = B * d.Wy;
+    t.Wa = d.Wy;  // per-coloring stride of the neighbours' dY rows
+    t.Wy = d.Wa;  // values per coloring: the aux child's row
+    t.Wo = d.Wa;
+    t.ymask = d.amask.as<uint16_t>();
+    t.xmask = d.ymask.as<uint16_t>();  // the set of each position of a neighbour's dY row (colour runs)
+    t.gidx = d.gidxT.as<int16_t>();
+    t.Wy4 = d.Wa4;
+    t.out = Ga;
+    t.ldo = B * d.Wa;
+    return t;
 }
 
 GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
@@ -1761,7 +1797,9 @@ GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
     }
     g.fwd.off_ykeep.assign(p->nsub, 0);
     for (auto& d : p->subs) {
-        if (!fused_grad_step(c, p, *d)) continue;
+        // Y kept for the steps without a gradient gather (which recomputes
+        // it), where the node launch reads it
+        if (!fused_grad_step(c, p, *d) && !(lane_grad_step(c, p, *d) && d->mm > 1)) continue;
         g.fwd.off_ykeep[d->s] = off;
         off += align_up((size_t)c->n_act * B * d->Wy * tsz, 256);
     }
@@ -1836,39 +1874,40 @@ int enqueue_sub_backward(pg_ctx* c, const pg_plan* p, const DevSub& d, int B, co
     // per-entry gradient read and written by each launch that adds to it.
     const double col = 4.0 * (double)c->n_act * B, Z = (double)c->nnz;
     const double Cs = d.root ? 0.0 : d.Cs, Cm = d.mm > 1 ? d.Cm : 0.0, Ca = d.Ca;
-    if (d.aa > 1 && Yk) {
+    const bool by_lane = lane_grad_step(c, p, d) && (Yk || d.mm == 1);
+    if (d.aa > 1 && (Yk || by_lane)) {
         // dY and G_main from G, the main row and the kept Y
         na.Y = Yk;
         na.part = 0;
         if (!dy_is_g) {
-            // reads G, the main row and Y, writes dY and G_main
-            record(c, node_name, col * (Cs + 2.0 * Ca + 2.0 * Cm), true);
+            // reads G, the main row and Y, writes dY and G_main (by lane: the
+            // byte model of the two node launches it stands for)
+            record(c, node_name,
+                   by_lane ? col * (Cs + Cm + Ca) * (na.Tm ? 2.0 : 1.0) : col * (Cs + 2.0 * Ca + 2.0 * Cm), true);
             HIP_TRY(c, launch_bwd_node<T>(na, c->num_cus, st));
             record(c, "", 0, false);
         }
-        SubArgs<T> t = base_args;
-        t.out_mode = OUT_Y;
-        if (c->weighted) t.w = fp32 ? (const T*)c->d_wT32.p : (const T*)c->d_wT64.p;
-        t.aux = dYin;
-        t.lda = B * d.Wy;
-        t.Wa = d.Wy;  // per-coloring stride of the neighbours' dY rows
-        t.Wy = d.Wa;  // values per coloring: the aux child's row
-        t.Wo = d.Wa;
-        t.ymask = d.amask.as<uint16_t>();
-        t.xmask = d.ymask.as<uint16_t>();  // the set of each position of a neighbour's dY row
-        t.gidx = d.gidxT.as<int16_t>();
-        t.Wy4 = d.Wa4;
-        t.out = Ga;
-        t.ldo = B * d.Wa;
+        SubArgs<T> t = transposed_args<T>(c, d, B, base_args, dYin, Ga);
+        if (by_lane) {
+            // the byte model of the step's two gathers (neighbours' T_aux and
+            // dY in, Y out; neighbours' dY in, G_aux out; the gradient), so
+            // that a call's algorithmic bytes do not depend on how many
+            // launches make them; it reads less
+            const StepBytes bytes{2.0 * csc_bytes(c), 2.0 * col * Ca + 16.0 * Z, col * 3.0 * Ca};
+            t.dy = Ta;
+            t.ldd = B * d.Wa;
+            t.grad = c->d_grad.as<double>() + c->nnz;  // of the transposed entries
+            return launch_gathering<T>(c, AUX_GATHER_TG, MAIN_LEAF, t, pb.part, B * d.Wa, bytes);
+        }
+        // reads the neighbours' dY, the own aux rows and the transposed
+        // entry ids, writes G_aux, reads and writes each entry's gradient
+        const StepBytes bytes{csc_bytes(c), col * Ca + 20.0 * Z, col * 2.0 * Ca};
         t.own = Ta;
         t.ldown = B * d.Wa;
         t.tr = c->d_tr.as<int32_t>();
         t.ttab = d.ttab.as<int16_t>();
         t.grad = c->d_grad.as<double>();
-        // reads the neighbours' dY, the own aux rows and the transposed
-        // entry ids, writes G_aux, reads and writes each entry's gradient
-        return launch_gathering<T>(c, AUX_GATHER_T, MAIN_LEAF, t, pb.part, B * d.Wa,
-                                   StepBytes{csc_bytes(c), col * Ca + 20.0 * Z, col * 2.0 * Ca},
+        return launch_gathering<T>(c, AUX_GATHER_T, MAIN_LEAF, t, pb.part, B * d.Wa, bytes,
                                    runs_used_per_mille(p, d, AUX_GATHER_T));
     }
     if (d.aa > 1) {
@@ -1905,20 +1944,7 @@ int enqueue_sub_backward(pg_ctx* c, const pg_plan* p, const DevSub& d, int B, co
             HIP_TRY(c, launch_bwd_node<T>(na, c->num_cus, st));
             record(c, "", 0, false);
         }
-        SubArgs<T> t = base_args;
-        t.out_mode = OUT_Y;
-        if (c->weighted) t.w = fp32 ? (const T*)c->d_wT32.p : (const T*)c->d_wT64.p;
-        t.aux = dYin;
-        t.lda = B * d.Wy;
-        t.Wa = d.Wy;  // per-coloring stride of the neighbours' dY rows
-        t.Wy = d.Wa;  // values per coloring: the aux child's row
-        t.Wo = d.Wa;
-        t.ymask = d.amask.as<uint16_t>();
-        t.xmask = d.ymask.as<uint16_t>();  // the set of each position of a neighbour's dY row (colour runs)
-        t.gidx = d.gidxT.as<int16_t>();
-        t.Wy4 = d.Wa4;
-        t.out = Ga;
-        t.ldo = B * d.Wa;
+        const SubArgs<T> t = transposed_args<T>(c, d, B, base_args, dYin, Ga);
         // reads the neighbours' dY, writes G_aux
         rc = launch_gathering<T>(c, AUX_GATHER_T, MAIN_LEAF, t, pb.part, B * d.Wa,
                                  StepBytes{csc_bytes(c), col * Ca, col * Ca}, runs_used_per_mille(p, d, AUX_GATHER_T));
@@ -2204,8 +2230,14 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         HIP_TRY(c, wT.alloc(c->nnz * tsz));
         HIP_TRY(c, launch_gather_weights<T>(wT.as<T>(), c->d_w32.as<float>(), c->d_tr.as<int32_t>(), c->nnz, c->stream));
     }
-    HIP_TRY(c, c->d_grad.alloc(std::max<int64_t>(c->nnz, 1) * 8));
-    HIP_TRY(c, launch_zero_f64(c->d_grad.as<double>(), c->nnz, c->stream));
+    // the entries' gradients and, where a transposed gather takes them in list
+    // order (AUX_GATHER_TG), those of their transposes
+    bool by_transpose = false;
+    for (auto& d : p->subs) by_transpose |= lane_grad_step(c, p, *d);
+    const int64_t n_acc = c->nnz * (by_transpose ? 2 : 1);
+    HIP_TRY(c, c->d_grad.alloc(std::max<int64_t>(n_acc, 1) * 8));
+    HIP_TRY(c, launch_zero_f64(c->d_grad.as<double>(), n_acc, c->stream));
+    const double* g_tr = by_transpose ? c->d_grad.as<double>() + c->nnz : nullptr;
     const uint8_t* d_in = nullptr;
     if (colors) {
         if ((size_t)ncol * c->n > c->d_colors_in.bytes) {
@@ -2302,15 +2334,17 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         const double factor = finish_raw(p, sizeof(T) == 4, flags, 1.0);
         if (grad_on_device) {
             if (sizeof(T) == 4)
-                HIP_TRY(c, launch_scatter_grad_f32((float*)grad, c->d_grad.as<double>(), c->d_ent.as<int32_t>(),
-                                                   c->nnz, factor, c->stream));
+                HIP_TRY(c, launch_scatter_grad<float>((float*)grad, c->d_grad.as<double>(), g_tr, c->d_tr.as<int32_t>(),
+                                                      c->d_ent.as<int32_t>(), c->nnz, factor, c->stream));
             else
-                HIP_TRY(c, launch_scatter_grad_f64((double*)grad, c->d_grad.as<double>(), c->d_ent.as<int32_t>(),
-                                                   c->nnz, factor, c->stream));
+                HIP_TRY(c, launch_scatter_grad<double>((double*)grad, c->d_grad.as<double>(), g_tr,
+                                                       c->d_tr.as<int32_t>(), c->d_ent.as<int32_t>(), c->nnz, factor,
+                                                       c->stream));
         } else {
             HIP_TRY(c, c->d_grad_out.alloc(std::max<int64_t>(c->nnz, 1) * 8));
-            HIP_TRY(c, launch_scatter_grad_f64(c->d_grad_out.as<double>(), c->d_grad.as<double>(),
-                                               c->d_ent.as<int32_t>(), c->nnz, factor, c->stream));
+            HIP_TRY(c, launch_scatter_grad<double>(c->d_grad_out.as<double>(), c->d_grad.as<double>(), g_tr,
+                                                   c->d_tr.as<int32_t>(), c->d_ent.as<int32_t>(), c->nnz, factor,
+                                                   c->stream));
             HIP_TRY(c, hipMemcpyAsync(grad, c->d_grad_out.p, c->nnz * 8, hipMemcpyDeviceToHost, c->stream));
         }
     }

@@ -66,7 +66,7 @@ __device__ __forceinline__ T aux_term(const SubArgs<T>& a, const int16_t* s_rank
         }
         return T(0);
     }
-    if (AUX == AUX_GATHER_T) {
+    if (AUX == AUX_GATHER_T || AUX == AUX_GATHER_TG) {
         if (!((amask >> cu) & 1u)) {
             const int idx = s_rank[squeeze_bit(amask, cu)];
             return a.aux[(int64_t)u * a.lda + aoff + idx];
@@ -81,7 +81,8 @@ __host__ __device__ constexpr size_t rank_lds_bytes(int K) { return (((size_t)2 
 // per-lane gathers of neighbour rows (through the rank table or the gather index table)
 __host__ __device__ constexpr bool gathers_rows(int aux)
 {
-    return aux == AUX_GATHER || aux == AUX_GATHER_T || aux == AUX_STAGED || aux == AUX_GATHER_G;
+    return aux == AUX_GATHER || aux == AUX_GATHER_T || aux == AUX_STAGED || aux == AUX_GATHER_G ||
+           aux == AUX_GATHER_TG;
 }
 // launches that stage the rank table (and, row-wise, the aux row masks) in LDS
 __host__ __device__ constexpr bool uses_rank(int aux) { return gathers_rows(aux) || aux == AUX_ROWS; }
@@ -93,7 +94,7 @@ __host__ __device__ constexpr bool walks_entries(int aux) { return uses_rank(aux
 template <typename T>
 __host__ __device__ size_t index_lds_bytes(int aux, const SubArgs<T>& a)
 {
-    if ((aux == AUX_GATHER || aux == AUX_STAGED || aux == AUX_GATHER_T || aux == AUX_GATHER_G) && a.gidx)
+    if (gathers_rows(aux) && a.gidx)
         return ((size_t)2 * (a.k + 1) * a.k * a.Wy4 + 15) & ~(size_t)15;
     if (aux == AUX_ROWS && a.xidx) return ((size_t)2 * a.k * a.k * a.Wa4 + 15) & ~(size_t)15;
     return !uses_rank(aux) ? 0
@@ -207,8 +208,7 @@ __global__ __launch_bounds__(kBlock) void k_sub(const SubArgs<T> a)
     const int cln = lane - grp * cl;
     const int ycopies = AUX == AUX_ROWS ? ng : 1;
     const size_t head = head_lds_bytes(AUX, a);
-    const bool use_gidx =
-        (AUX == AUX_GATHER || AUX == AUX_STAGED || AUX == AUX_GATHER_T || AUX == AUX_GATHER_G) && a.gidx != nullptr;
+    const bool use_gidx = gathers_rows(AUX) && a.gidx != nullptr;
     constexpr bool staged = AUX == AUX_STAGED;
     static_assert(RC == kRegCols || gathers_rows(AUX), "one value per lane is a gather layout");
     const bool y_in_lds = !(mode == OUT_Y || mode == OUT_PARTIAL) || AUX == AUX_ROWS;
@@ -381,13 +381,15 @@ __global__ __launch_bounds__(kBlock) void k_sub(const SubArgs<T> a)
                     const bool ok = sv && i < W;
                     if (AUX == AUX_GATHER || AUX == AUX_GATHER_G) amask[r] = ok ? expand_bit(a.ymask[i], cv) : 0u;
                     else if (AUX == AUX_STAGED) amask[r] = 0u;  // the gather index table replaces it
-                    else if (AUX == AUX_GATHER_T) amask[r] = ok ? expand_bit(a.ymask[i], cv) | (1u << cv) : ~0u;
+                    else if (AUX == AUX_GATHER_T || AUX == AUX_GATHER_TG)
+                        amask[r] = ok ? expand_bit(a.ymask[i], cv) | (1u << cv) : ~0u;
                     else amask[r] = ok ? (uint32_t)i : 0xffu;
                 }
                 const int aoff = b * a.Wa;
-                // adjoint: this slot's dY values (zero past the row's end)
+                // adjoint: this slot's dY values (of the vertex's own aux row
+                // where the neighbours' rows are dY), zero past the row's end
                 T dyv[RC];
-                constexpr bool edge_grad = AUX == AUX_GATHER_G;
+                constexpr bool edge_grad = AUX == AUX_GATHER_G || AUX == AUX_GATHER_TG;
                 if (edge_grad)
 #pragma unroll
                     for (int r = 0; r < RC; ++r)
@@ -715,7 +717,7 @@ static hipError_t launch_one(const SubArgs<T>& a, int num_cus, int blocks_per_cu
 template <typename T, int TEAM, int AUX, int MAIN>
 static hipError_t launch_rc(int rc, const SubArgs<T>& a, int num_cus, int per_cu, hipStream_t st)
 {
-    if constexpr (AUX == AUX_GATHER || AUX == AUX_GATHER_G || AUX == AUX_GATHER_T) {
+    if constexpr (AUX == AUX_GATHER || AUX == AUX_GATHER_G || AUX == AUX_GATHER_T || AUX == AUX_GATHER_TG) {
         if (rc == 1) return launch_one<T, TEAM, AUX, MAIN, 1>(a, num_cus, per_cu, st);
     }
     if (rc != kRegCols) return hipErrorInvalidValue;
@@ -733,6 +735,7 @@ static hipError_t launch_team(int aux, int main_mode, int rc, const SubArgs<T>& 
         case AUX_STAGED: return launch_rc<T, TEAM, AUX_STAGED, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
         case AUX_GATHER_G: return launch_rc<T, TEAM, AUX_GATHER_G, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
         case AUX_GATHER_T: return launch_rc<T, TEAM, AUX_GATHER_T, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
+        case AUX_GATHER_TG: return launch_rc<T, TEAM, AUX_GATHER_TG, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
         case AUX_COLORS: return launch_rc<T, TEAM, AUX_COLORS, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
         case AUX_READ: return launch_rc<T, TEAM, AUX_READ, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
         case AUX_PARTIALS: return launch_rc<T, TEAM, AUX_PARTIALS, MAIN_LEAF>(rc, a, num_cus, per_cu, st);
@@ -1396,28 +1399,29 @@ template hipError_t launch_edge_grad<float>(const EdgeGradArgs<float>&, hipStrea
 template hipError_t launch_edge_grad<double>(const EdgeGradArgs<double>&, hipStream_t);
 
 template <typename TO>
-__global__ void k_scatter_grad(TO* out, const double* grad, const int32_t* ent, int64_t nnz, double factor)
+__global__ void k_scatter_grad(TO* out, const double* grad, const double* grad_tr, const int32_t* tr,
+                               const int32_t* ent, int64_t nnz, double factor)
 {
-    FLAT_LOOP(i, nnz) out[ent[i]] = (TO)(factor * grad[i]);
+    if (grad_tr) {
+        FLAT_LOOP(i, nnz) out[ent[i]] = (TO)((grad[i] + grad_tr[tr[i]]) * factor);
+    } else {
+        FLAT_LOOP(i, nnz) out[ent[i]] = (TO)(grad[i] * factor);
+    }
 }
 
-hipError_t launch_scatter_grad_f32(float* out, const double* grad, const int32_t* ent, int64_t nnz, double factor,
-                                   hipStream_t st)
+template <typename TO>
+hipError_t launch_scatter_grad(TO* out, const double* grad, const double* grad_tr, const int32_t* tr, const int32_t* ent,
+                               int64_t nnz, double factor, hipStream_t st)
 {
     if (nnz == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter_grad<float>, flat_grid(nnz), dim3(256), 0, st, out, grad, ent,
-                       nnz, factor);
+    hipLaunchKernelGGL(k_scatter_grad<TO>, flat_grid(nnz), dim3(256), 0, st, out, grad, grad_tr, tr, ent, nnz, factor);
     return hipGetLastError();
 }
 
-hipError_t launch_scatter_grad_f64(double* out, const double* grad, const int32_t* ent, int64_t nnz, double factor,
-                                   hipStream_t st)
-{
-    if (nnz == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter_grad<double>, flat_grid(nnz), dim3(256), 0, st, out, grad, ent,
-                       nnz, factor);
-    return hipGetLastError();
-}
+template hipError_t launch_scatter_grad<float>(float*, const double*, const double*, const int32_t*, const int32_t*,
+                                               int64_t, double, hipStream_t);
+template hipError_t launch_scatter_grad<double>(double*, const double*, const double*, const int32_t*, const int32_t*,
+                                                int64_t, double, hipStream_t);
 
 __global__ void k_zero_f64(double* p, int64_t n)
 {

@@ -30,6 +30,9 @@ enum AuxMode : int {
     AUX_STAGED = 6,    // AUX_GATHER through the gather index table with neighbour rows staged in
                        // LDS (needs SubArgs::gidx and segpad)
     AUX_GATHER_G = 7,  // AUX_GATHER of the adjoint: also grad[e] += dY . x_e per entry (needs dy, grad)
+    AUX_GATHER_TG = 8, // AUX_GATHER_T that also takes the gradients: grad[e] += dy . x_e, where dy is the
+                       // vertex's own aux row and x_e what the neighbour's dY row adds to it: the
+                       // derivative of the transposed entry
 };
 // Where the main-child values come from.
 enum MainMode : int {
@@ -110,6 +113,7 @@ struct SubArgs {
     // AUX_GATHER_G: each neighbour's contribution x to the vertex's Y row is
     // also contracted with dY there, and grad[e] += sum over the row of dY * x
     // (in FP64) for the entry e
+    // (AUX_GATHER_TG: dy holds the vertices' own aux rows)
     const T* dy;             // [n_act][ldd]
     int32_t ldd;             // dy row stride (B * Wy)
     double* grad;            // [nnz] internal entry order
@@ -278,11 +282,10 @@ struct EdgeGradArgs {
 template <typename T>
 hipError_t launch_edge_grad(const EdgeGradArgs<T>& a, hipStream_t st);
 
-// out[ent[i]] (=/+=) (TO) (factor * grad[i])
-hipError_t launch_scatter_grad_f32(float* out, const double* grad, const int32_t* ent, int64_t nnz, double factor,
-                                   hipStream_t st);
-hipError_t launch_scatter_grad_f64(double* out, const double* grad, const int32_t* ent, int64_t nnz, double factor,
-                                   hipStream_t st);
+// out[ent[i]] = (TO) (factor * (grad[i] + grad_tr[tr[i]])); grad_tr nullptr: grad alone
+template <typename TO>
+hipError_t launch_scatter_grad(TO* out, const double* grad, const double* grad_tr, const int32_t* tr, const int32_t* ent,
+                               int64_t nnz, double factor, hipStream_t st);
 hipError_t launch_zero_f64(double* p, int64_t n, hipStream_t st);
 
 // ---- the reference's unpruned mode (isPruned = 0, CountMat.cpp:851-977) ----
