@@ -126,6 +126,10 @@ constexpr size_t kGidxMaxBytes = 24 * 1024;
 // list of 4096 entries takes 4 wavefronts some 50 us, as long as a gathering
 // step's other launch takes on the smallest graphs with such hubs
 constexpr int64_t kHubBigDegree = 4096;
+// colorings per pass up to which the root takes k_root_seq, which handles four at
+// a time: with more, the gathering kernel is as fast (5 colorings, FP64, uniform
+// graph: 0.38 ms by tiles, 0.35 by teams) or faster (64, scale 20: 4.4 against 2.0)
+constexpr int kRootTileColorings = 4;
 
 }  // namespace
 
@@ -188,6 +192,8 @@ struct pg_ctx {
     int32_t n_hub_items = 0, n_slots = 0;
     int32_t n_big = 0;  // leading hubs above kHubBigDegree: k_hub_seq gives them a whole workgroup
     DevBuf d_hub_items, d_slot_begin;
+    DevBuf d_root_tiles;  // tiles of the vertices below the hubs for k_root_seq
+    int n_root_tiles = 0;
     DevBuf d_hub_iota;  // [n_hub+1] h -> h: one partial row per hub (column-split hub launches)
     // per-call workspace
     DevBuf d_arena, d_colors_in;
@@ -308,6 +314,20 @@ int build_buckets(pg_ctx* c)
         std::iota(iota.begin(), iota.end(), 0);
         HIP_TRY(c, c->d_hub_iota.alloc(iota.size() * sizeof(int32_t)));
         HIP_TRY(c, hipMemcpy(c->d_hub_iota.p, iota.data(), iota.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    }
+    {
+        std::vector<int4> tiles;
+        for (int32_t v = nh; v < c->n_act;) {
+            const int32_t e = c->h_rowptr[v];
+            int32_t w = v + 1;
+            while (w < c->n_act && w - v < kRootTileVertices && c->h_rowptr[w + 1] - e <= kRootTileEntries) ++w;
+            tiles.push_back(make_int4(v, w - v, e, c->h_rowptr[w] - e));
+            v = w;
+        }
+        c->n_root_tiles = (int)tiles.size();
+        HIP_TRY(c, c->d_root_tiles.alloc(std::max<size_t>(tiles.size(), 1) * sizeof(int4)));
+        if (!tiles.empty())
+            HIP_TRY(c, hipMemcpy(c->d_root_tiles.p, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
     }
     drop_graphs(c);  // captured passes hold the old bucket ranges
     c->generation++;
@@ -868,6 +888,9 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         if (N > 0) b += bytes.per_vertex * verts / N;
         return b;
     };
+    // a root with one value per vertex and coloring, few colorings
+    const bool root_tiles =
+        a.Wy == 1 && a.B <= kRootTileColorings && a.out_mode == OUT_ROOT && main_mode == MAIN_LEAF && a.gidx && !a.ykeep;
     a.ng = 1;
     auto hubs = [&](hipStream_t hs) -> int {
         SubArgs<T> h = a;
@@ -890,7 +913,10 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         r.item_base = c->n_hub;
         r.n_items = c->n_act - c->n_hub;
         const double sh = share((double)c->nnz - c->h_rowptr[c->n_hub], c->n_act - c->n_hub);
-        if (rows) {
+        if (root_tiles) {
+            record(c, sizeof(T) == 4 ? "k_root_seq<float>" : "k_root_seq<double>", sh, true);
+            HIP_TRY(c, launch_root_seq<T>(r, c->d_root_tiles.as<int4>(), c->n_root_tiles, cus, rs));
+        } else if (rows) {
             record(c, runs_name(sizeof(T), RUNS_SEQ, main_mode), sh, true);
             HIP_TRY(c, launch_runs<T>(RUNS_SEQ, main_mode, r, cus, c->blocks_per_cu, rs));
         } else {

@@ -206,6 +206,14 @@ size_t hub_seq_lds_bytes(int k);
 template <typename T>
 hipError_t launch_hub_seq(const SubArgs<T>& a, int n_big, hipStream_t st);
 
+// The root's sums in the reference's order (GATHER, OUT_ROOT, main a leaf: one
+// value per vertex and coloring) for tiles {first vertex, vertices, first
+// entry, entries}: consecutive vertices within the two limits, or one vertex
+// with any number of entries (pg_root.hip).
+constexpr int kRootTileEntries = 1024, kRootTileVertices = kBlock;
+template <typename T>
+hipError_t launch_root_seq(const SubArgs<T>& a, const int4* tiles, int n_tiles, int num_cus, hipStream_t st);
+
 // Per-pass values read from device memory, so that one captured graph serves
 // every pass of the same shape (the host writes them before each replay).
 struct PassParams {

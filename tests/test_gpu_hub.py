@@ -1,7 +1,9 @@
 """The hub kernel's neighbour lists at the lengths where it can go wrong:
 around its batches of entries, around the turns of 4 and of 16 wavefronts, and
 around the degree from which a hub takes a whole workgroup; rows narrower and
-wider than a wavefront, one coloring per wavefront and several packed."""
+wider than a wavefront, one coloring per wavefront and several packed.  With
+fewer hubs the same lists go through the other vertices' kernels: the root's
+tiles (of 1,024 entries and 256 vertices, a longer list in windows) among them."""
 import numpy as np
 import pytest
 
@@ -39,14 +41,15 @@ def _graph():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hub_degree", [16, 600, 1 << 30])
 @pytest.mark.parametrize("k,edges,colorings", [
-    (3, U3, (1, 2, 33)),       # rows of one value: up to 32 colorings a wavefront
-    (5, U5, (1, 5, 16)),       # rows of 4 and 6 values
+    (3, U3, (1, 2, 3, 4, 5, 33)),  # rows of one value: up to 32 colorings a wavefront
+    (5, U5, (1, 4, 5, 16)),    # rows of 4 and 6 values
     (6, STAR6, (3,)),
     (7, TREE7, (1, 3, 10)),    # rows of 6, 15 and 20 values
     (10, TREE10, (1, 4)),      # rows of 9 to 126 values: two wavefronts each
 ])
-def test_hub_lists_keep_the_reference_arithmetic(gpu_ctx, k, edges, colorings):
+def test_hub_lists_keep_the_reference_arithmetic(gpu_ctx, k, edges, colorings, hub_degree):
     """FP32 counts equal the oracle's restatement of the reference up to the
     order of the final FP64 sum over 12,000 vertices (12,000 * 2^-53 < 2e-12
     relative for a sum of non-negative terms); FP64 counts below 2^53 are
@@ -56,7 +59,7 @@ def test_hub_lists_keep_the_reference_arithmetic(gpu_ctx, k, edges, colorings):
     keys = ("hub_degree", "exact_order")
     saved = [gpu_ctx.get_option(key) for key in keys]
     try:
-        gpu_ctx.set_option("hub_degree", 16)
+        gpu_ctx.set_option("hub_degree", hub_degree)
         gpu_ctx.set_option("exact_order", 1)
         rng = np.random.default_rng(43 + k)
         weights = rng.uniform(0.5, 1.5, len(rowidx)).astype(np.float32)
