@@ -697,10 +697,10 @@ std::string runs_name(size_t tsz, int mode, int main_mode)
 // process down in the runtime there; those branches already run side by
 // side).
 template <typename H, typename R>
-int fork_hubs(pg_ctx* c, bool have_hubs, H hubs, R rest)
+int fork_hubs(pg_ctx* c, bool have_hubs, H hubs, R rest, bool fork = true)
 {
     if (!have_hubs) return rest(c->stream);
-    if (!c->hub_concurrent || c->timing || !c->hub_stream || c->in_branches) {
+    if (!fork || !c->hub_concurrent || c->timing || !c->hub_stream || c->in_branches) {
         const int rc = hubs(c->stream);
         return rc ? rc : rest(c->stream);
     }
@@ -841,7 +841,9 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         }
         return PG_OK;
     };
-    const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest);
+    // (a histogram over few entries takes less than the fork and join)
+    const bool fork = aux != AUX_COLORS || (double)c->nnz * a.B > (1 << 22);
+    const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest, fork);
     if (frc) return frc;
     if (c->n_hub > 0) {
         SubArgs<T> f = a;
@@ -926,7 +928,17 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         record(c, "", 0, false);
         return PG_OK;
     };
-    const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest);
+    // Side by side unless that gains nothing: where the longest list's chain
+    // (4.4 ns an entry) is less than a twentieth of the hub launch's work (0.037
+    // ns per entry and wavefront unit), the two launches only compete (7-vertex
+    // tree, R-MAT scale 20, 64 colorings: 42.1 ms side by side, 39.2 ms one after
+    // the other); and where the other launch is a root's over few entries, a
+    // fork and join cost more than it takes (3-path, scale 16: 162 against 152
+    // us).
+    const double hub_work = 0.037 * c->h_rowptr[c->n_hub] * ((a.B * (double)a.Wy + 63) / 64);
+    const double rest_entries = ((double)c->nnz - c->h_rowptr[c->n_hub]) * a.B;
+    const bool fork = (a.Wy > 48 || 4.4 * c->max_deg > 0.05 * hub_work) && (!root_tiles || rest_entries > (1 << 21));
+    const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest, fork);
     if (frc) return frc;
     if (c->n_hub > 0) {
         SubArgs<T> f = a;
