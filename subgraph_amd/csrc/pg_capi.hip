@@ -194,6 +194,8 @@ struct pg_ctx {
     DevBuf d_hub_items, d_slot_begin;
     DevBuf d_root_tiles;  // tiles of the vertices below the hubs for k_root_seq
     int n_root_tiles = 0;
+    DevBuf d_stream_tiles, d_local;  // and for k_stream, with each entry's vertex in its tile
+    int n_stream_tiles = 0;
     DevBuf d_hub_iota;  // [n_hub+1] h -> h: one partial row per hub (column-split hub launches)
     // per-call workspace
     DevBuf d_arena, d_colors_in;
@@ -315,20 +317,28 @@ int build_buckets(pg_ctx* c)
         HIP_TRY(c, c->d_hub_iota.alloc(iota.size() * sizeof(int32_t)));
         HIP_TRY(c, hipMemcpy(c->d_hub_iota.p, iota.data(), iota.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     }
-    {
+    // tiles of the vertices below the hubs: consecutive ones within both limits
+    auto make_tiles = [&](int max_entries, int max_vertices, DevBuf& buf, int& n) -> int {
         std::vector<int4> tiles;
         for (int32_t v = nh; v < c->n_act;) {
             const int32_t e = c->h_rowptr[v];
             int32_t w = v + 1;
-            while (w < c->n_act && w - v < kRootTileVertices && c->h_rowptr[w + 1] - e <= kRootTileEntries) ++w;
+            while (w < c->n_act && w - v < max_vertices && c->h_rowptr[w + 1] - e <= max_entries) ++w;
             tiles.push_back(make_int4(v, w - v, e, c->h_rowptr[w] - e));
             v = w;
         }
-        c->n_root_tiles = (int)tiles.size();
-        HIP_TRY(c, c->d_root_tiles.alloc(std::max<size_t>(tiles.size(), 1) * sizeof(int4)));
-        if (!tiles.empty())
-            HIP_TRY(c, hipMemcpy(c->d_root_tiles.p, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
-    }
+        n = (int)tiles.size();
+        HIP_TRY(c, buf.alloc(std::max<size_t>(tiles.size(), 1) * sizeof(int4)));
+        if (!tiles.empty()) HIP_TRY(c, hipMemcpy(buf.p, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
+        return PG_OK;
+    };
+    int rc = make_tiles(kRootTileEntries, kRootTileVertices, c->d_root_tiles, c->n_root_tiles);
+    if (rc) return rc;
+    rc = make_tiles(kStreamTileEntries, kStreamTileVertices, c->d_stream_tiles, c->n_stream_tiles);
+    if (rc) return rc;
+    HIP_TRY(c, c->d_local.alloc(std::max<int64_t>(c->nnz, 1)));
+    HIP_TRY(c, launch_local_ids(c->d_local.as<uint8_t>(), c->d_stream_tiles.as<int4>(), c->n_stream_tiles,
+                                c->d_rowptr.as<int32_t>(), c->stream));
     drop_graphs(c);  // captured passes hold the old bucket ranges
     c->generation++;
     c->built_deg = c->hub_degree;
@@ -893,6 +903,21 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
     // a root with one value per vertex and coloring, few colorings
     const bool root_tiles =
         a.Wy == 1 && a.B <= kRootTileColorings && a.out_mode == OUT_ROOT && main_mode == MAIN_LEAF && a.gidx && !a.ykeep;
+    // Narrow rows loaded whole and permuted (k_stream) against k_sub's permuted
+    // loads: always where the rows are no wider than the sums; where they are
+    // wider it loads more than it uses, and gains while it needs few chunks of
+    // colorings.  R-MAT scale 18, ms by k_stream / k_sub, rows -> sums: 1
+    // coloring 15 -> 20 0.10 / 0.18; 4 colorings 28 -> 8 0.21 / 0.30 (2 chunks),
+    // 56 -> 28 0.43 / 0.51 (4), 36 -> 9 0.42 / 0.30 (4); 16 colorings 6 -> 4
+    // 0.21 / 0.25 (2), 15 -> 6 0.44 / 0.52 (4), 20 -> 15 0.76 / 0.77 (6), 21 -> 7
+    // 0.80 / 0.63 (6), 35 -> 21 1.64 / 1.43 (16), 9 -> 36 1.5 / 1.8.
+    bool stream = false;
+    if constexpr (sizeof(T) == 4)
+        if (!rows && main_mode == MAIN_LEAF && (a.out_mode == OUT_EMA || a.out_mode == OUT_EMA_SCALED) && a.gidx &&
+            a.Wy <= 64 && a.Wa <= 63 && (int64_t)c->n_act * a.lda * 4 < ((int64_t)1 << 32) - 16) {
+            const int chunks = (a.B + stream_colorings(a) - 1) / stream_colorings(a);
+            stream = a.Wa <= a.Wy || chunks <= 2 || (chunks <= 4 && a.Wa <= 3 * a.Wy);
+        }
     a.ng = 1;
     auto hubs = [&](hipStream_t hs) -> int {
         SubArgs<T> h = a;
@@ -915,7 +940,13 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         r.item_base = c->n_hub;
         r.n_items = c->n_act - c->n_hub;
         const double sh = share((double)c->nnz - c->h_rowptr[c->n_hub], c->n_act - c->n_hub);
-        if (root_tiles) {
+        if (stream) {
+            if constexpr (sizeof(T) == 4) {
+                record(c, "k_stream<float>", sh, true);
+                HIP_TRY(c, launch_stream(r, c->d_stream_tiles.as<int4>(), c->n_stream_tiles, c->d_local.as<uint8_t>(),
+                                         c->n_act, cus, rs));
+            }
+        } else if (root_tiles) {
             record(c, sizeof(T) == 4 ? "k_root_seq<float>" : "k_root_seq<double>", sh, true);
             HIP_TRY(c, launch_root_seq<T>(r, c->d_root_tiles.as<int4>(), c->n_root_tiles, cus, rs));
         } else if (rows) {
