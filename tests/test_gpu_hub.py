@@ -14,6 +14,7 @@ TREE7 = [(0, 1), (1, 2), (2, 3), (1, 4), (4, 5), (4, 6)]
 TREE10 = [(0, 1), (1, 2), (2, 3), (3, 4), (1, 5), (5, 6), (5, 7), (7, 8), (7, 9)]
 U3 = [(0, 1), (1, 2)]
 U5 = [(0, 1), (1, 2), (2, 3), (3, 4)]
+PATH12 = [(i, i + 1) for i in range(11)]
 STAR6 = [(0, 1), (1, 2), (1, 3), (1, 4), (1, 5)]
 # list lengths: one batch (32 FP64, 56 FP32 entries) and its neighbours, whole
 # rounds of 4 and 16 wavefronts, the whole-workgroup degree, a long list
@@ -48,6 +49,7 @@ def _graph():
     (6, STAR6, (3,)),
     (7, TREE7, (1, 3, 10)),    # rows of 6, 15 and 20 values
     (10, TREE10, (1, 4)),      # rows of 9 to 126 values: two wavefronts each
+    (12, PATH12, (2,)),        # rows of up to 462 values: eight, a unit of all hubs at a time
 ])
 def test_hub_lists_keep_the_reference_arithmetic(gpu_ctx, k, edges, colorings, hub_degree):
     """FP32 counts equal the oracle's restatement of the reference up to the
