@@ -196,6 +196,7 @@ struct pg_ctx {
     int n_root_tiles = 0;
     DevBuf d_stream_tiles, d_local;  // and for k_stream, with each entry's vertex in its tile
     int n_stream_tiles = 0;
+    std::vector<int32_t> h_stream_first;  // each tile's first vertex
     DevBuf d_hub_iota;  // [n_hub+1] h -> h: one partial row per hub (column-split hub launches)
     // per-call workspace
     DevBuf d_arena, d_colors_in;
@@ -318,13 +319,14 @@ int build_buckets(pg_ctx* c)
         HIP_TRY(c, hipMemcpy(c->d_hub_iota.p, iota.data(), iota.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     }
     // tiles of the vertices below the hubs: consecutive ones within both limits
-    auto make_tiles = [&](int max_entries, int max_vertices, DevBuf& buf, int& n) -> int {
+    auto make_tiles = [&](int max_entries, int max_vertices, DevBuf& buf, int& n, std::vector<int32_t>* first) -> int {
         std::vector<int4> tiles;
         for (int32_t v = nh; v < c->n_act;) {
             const int32_t e = c->h_rowptr[v];
             int32_t w = v + 1;
             while (w < c->n_act && w - v < max_vertices && c->h_rowptr[w + 1] - e <= max_entries) ++w;
             tiles.push_back(make_int4(v, w - v, e, c->h_rowptr[w] - e));
+            if (first) first->push_back(v);
             v = w;
         }
         n = (int)tiles.size();
@@ -332,9 +334,10 @@ int build_buckets(pg_ctx* c)
         if (!tiles.empty()) HIP_TRY(c, hipMemcpy(buf.p, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
         return PG_OK;
     };
-    int rc = make_tiles(kRootTileEntries, kRootTileVertices, c->d_root_tiles, c->n_root_tiles);
+    int rc = make_tiles(kRootTileEntries, kRootTileVertices, c->d_root_tiles, c->n_root_tiles, nullptr);
     if (rc) return rc;
-    rc = make_tiles(kStreamTileEntries, kStreamTileVertices, c->d_stream_tiles, c->n_stream_tiles);
+    c->h_stream_first.clear();
+    rc = make_tiles(kStreamTileEntries, kStreamTileVertices, c->d_stream_tiles, c->n_stream_tiles, &c->h_stream_first);
     if (rc) return rc;
     HIP_TRY(c, c->d_local.alloc(std::max<int64_t>(c->nnz, 1)));
     HIP_TRY(c, launch_local_ids(c->d_local.as<uint8_t>(), c->d_stream_tiles.as<int4>(), c->n_stream_tiles,
@@ -882,6 +885,31 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
 //    neighbour group, by whole rows (RUNS_SEQ, when `rows`) or by gathers;
 //  - the finishing launch adds each hub's single partial row to zero and
 //    combines it with the main table.
+// the first streaming tile that starts at vertex v or later, and the last
+// vertex in [v0, v] that starts a tile (v itself where the tiles end)
+int tile_of(const pg_ctx* c, int32_t v)
+{
+    const auto& f = c->h_stream_first;
+    return (int)(std::lower_bound(f.begin(), f.end(), v) - f.begin());
+}
+
+int32_t tile_floor(const pg_ctx* c, int32_t v0, int32_t v)
+{
+    const auto& f = c->h_stream_first;
+    if (v >= c->n_act) return v;
+    const auto it = std::upper_bound(f.begin(), f.end(), v);
+    return it == f.begin() ? v0 : std::max(v0, *(it - 1));
+}
+
+// The combine apart from the gather pays from this many products per value of
+// the rows: steps of 6.8 (12-vertex tree, R-MAT scale 20, 4 colorings) 12.6 ->
+// 8.1 ms and 7.9 -> 4.4, of 2.3 (10-vertex tree, scale 18, 4 colorings) 1.61 ->
+// 1.50; of 1.5 (7-vertex tree, scale 20) 8.5 -> 8.7 ms with 64 colorings and
+// 0.21 -> 0.50 with one.  And for a part of this many rows: below, its two
+// launches and the drain between them cost more than they save.
+constexpr int64_t kCombineReuse = 2;
+constexpr int64_t kCombineRowsMin = 1 << 14;
+
 template <typename T>
 int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, int y_cols, StepBytes bytes,
                            bool rows)
@@ -903,6 +931,14 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
     // a root with one value per vertex and coloring, few colorings
     const bool root_tiles =
         a.Wy == 1 && a.B <= kRootTileColorings && a.out_mode == OUT_ROOT && main_mode == MAIN_LEAF && a.gidx && !a.ykeep;
+    // Y rows to memory and the combine a launch of its own (k_combine_rows)
+    bool by_rows = false;
+    if constexpr (sizeof(T) == 4)
+        by_rows = main_mode == MAIN_TABLE && a.out_mode == OUT_EMA && a.ldo == a.B * a.Wo && a.ldm == a.B * a.Wm &&
+                  (!a.ykeep || a.ldy == a.B * a.Wy) && a.Wy < 1024 && a.Wm < 1024 &&
+                  combine_rows_lds_bytes(a.Wy, a.Wm, a.Wo, a.P) <= kLdsLimit &&
+                  (int64_t)a.P * a.Wo >= kCombineReuse * (a.Wy + a.Wm + a.Wo);
+    const int gather_main = by_rows ? MAIN_LEAF : main_mode;  // the gather's own outputs: Y
     // Narrow rows loaded whole and permuted (k_stream) against k_sub's permuted
     // loads: always where the rows are no wider than the sums; where they are
     // wider it loads more than it uses, and gains while it needs few chunks of
@@ -913,7 +949,7 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
     // 0.80 / 0.63 (6), 35 -> 21 1.64 / 1.43 (16), 9 -> 36 1.5 / 1.8.
     bool stream = false;
     if constexpr (sizeof(T) == 4)
-        if (!rows && main_mode == MAIN_LEAF && (a.out_mode == OUT_EMA || a.out_mode == OUT_EMA_SCALED) && a.gidx &&
+        if (!rows && gather_main == MAIN_LEAF && (a.out_mode == OUT_EMA || a.out_mode == OUT_EMA_SCALED) && a.gidx &&
             a.Wy <= 64 && a.Wa <= 63 && (int64_t)c->n_act * a.lda * 4 < ((int64_t)1 << 32) - 16) {
             const int chunks = (a.B + stream_colorings(a) - 1) / stream_colorings(a);
             stream = a.Wa <= a.Wy || chunks <= 2 || (chunks <= 4 && a.Wa <= 3 * a.Wy);
@@ -933,31 +969,67 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         record(c, "", 0, false);
         return PG_OK;
     };
-    auto rest = [&](hipStream_t rs) -> int {
-        if (c->n_hub >= c->n_act) return PG_OK;
-        SubArgs<T> r = a;
+    // vertices [v0, v1) below the hubs
+    auto gather = [&](SubArgs<T> r, int32_t v0, int32_t v1, int mm, bool streamed, hipStream_t rs) -> int {
         r.items = nullptr;
-        r.item_base = c->n_hub;
-        r.n_items = c->n_act - c->n_hub;
-        const double sh = share((double)c->nnz - c->h_rowptr[c->n_hub], c->n_act - c->n_hub);
-        if (stream) {
+        r.item_base = v0;
+        r.n_items = v1 - v0;
+        const double sh = share((double)c->h_rowptr[v1] - c->h_rowptr[v0], by_rows && mm != main_mode ? 0 : v1 - v0);
+        if (streamed) {
             if constexpr (sizeof(T) == 4) {
+                const int t0 = tile_of(c, v0), t1 = tile_of(c, v1);
                 record(c, "k_stream<float>", sh, true);
-                HIP_TRY(c, launch_stream(r, c->d_stream_tiles.as<int4>(), c->n_stream_tiles, c->d_local.as<uint8_t>(),
+                HIP_TRY(c, launch_stream(r, c->d_stream_tiles.as<int4>() + t0, t1 - t0, c->d_local.as<uint8_t>(),
                                          c->n_act, cus, rs));
             }
         } else if (root_tiles) {
             record(c, sizeof(T) == 4 ? "k_root_seq<float>" : "k_root_seq<double>", sh, true);
             HIP_TRY(c, launch_root_seq<T>(r, c->d_root_tiles.as<int4>(), c->n_root_tiles, cus, rs));
         } else if (rows) {
-            record(c, runs_name(sizeof(T), RUNS_SEQ, main_mode), sh, true);
-            HIP_TRY(c, launch_runs<T>(RUNS_SEQ, main_mode, r, cus, c->blocks_per_cu, rs));
+            record(c, runs_name(sizeof(T), RUNS_SEQ, mm), sh, true);
+            HIP_TRY(c, launch_runs<T>(RUNS_SEQ, mm, r, cus, c->blocks_per_cu, rs));
         } else {
-            record(c, kname<T>(cl, aux_b, main_mode, rc), sh, true);
-            HIP_TRY(c, launch_sub<T>(cl, aux_b, main_mode, rc, r, cus, c->blocks_per_cu, rs));
+            record(c, kname<T>(cl, aux_b, mm, rc), sh, true);
+            HIP_TRY(c, launch_sub<T>(cl, aux_b, mm, rc, r, cus, c->blocks_per_cu, rs));
         }
         record(c, "", 0, false);
         return PG_OK;
+    };
+    auto rest = [&](hipStream_t rs) -> int {
+        if (c->n_hub >= c->n_act) return PG_OK;
+        if constexpr (sizeof(T) == 4) {
+            SubArgs<T> r = a;
+            r.main = nullptr;
+            r.ykeep = nullptr;
+            r.Wo = a.Wy;
+            r.P = 0;
+            r.split_lds = 0;
+            r.ldo = a.B * a.Wy;
+            for (int32_t v = c->n_hub; by_rows && v < c->n_act;) {
+                // Y goes where it is kept or, a part of the vertices at a time,
+                // to the output table's rows past that part, which are not
+                // written yet; the last few go the fused way
+                int32_t end = c->n_act;
+                T* y = a.ykeep;
+                if (!y) {
+                    end = v + (int32_t)((int64_t)(c->n_act - v) * a.Wo / (a.Wo + a.Wy));
+                    if (stream) end = tile_floor(c, v, end);
+                    if ((int64_t)(end - v) * a.B < kCombineRowsMin) return gather(a, v, c->n_act, main_mode, false, rs);
+                    y = a.out + (int64_t)end * a.ldo - (int64_t)v * r.ldo;
+                }
+                r.out = y;
+                int rc = gather(r, v, end, MAIN_LEAF, stream, rs);
+                if (rc) return rc;
+                record(c, "k_combine_rows<float>", share(0, end - v), true);
+                HIP_TRY(c, launch_combine_rows(y + (int64_t)v * r.ldo, a.main + (int64_t)v * a.ldm,
+                                               a.out + (int64_t)v * a.ldo, a.split, (int64_t)(end - v) * a.B, a.Wy,
+                                               a.Wm, a.Wo, a.P, cus, rs));
+                record(c, "", 0, false);
+                v = end;
+            }
+            if (by_rows) return PG_OK;
+        }
+        return gather(a, c->n_hub, c->n_act, main_mode, stream, rs);
     };
     // Side by side unless that gains nothing: where the longest list's chain
     // (4.4 ns an entry) is less than a twentieth of the hub launch's work (0.037

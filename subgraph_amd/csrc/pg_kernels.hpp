@@ -225,6 +225,13 @@ hipError_t launch_stream(const SubArgs<float>& a, const int4* tiles, int n_tiles
                          int num_cus, hipStream_t st);
 hipError_t launch_local_ids(uint8_t* local, const int4* tiles, int n_tiles, const int32_t* rowptr, hipStream_t st);
 
+// The combine of n FP32 rows whose Y is in memory (pg_combine.hip): dense rows
+// y[n][Wy] and m[n][Wm] into out[n][Wo] by the split table [Wo][P], OUT_EMA.
+constexpr int kCombineRows = 16;
+size_t combine_rows_lds_bytes(int Wy, int Wm, int Wo, int P);
+hipError_t launch_combine_rows(const float* y, const float* m, float* out, const uint32_t* split, int64_t n, int Wy,
+                               int Wm, int Wo, int P, int num_cus, hipStream_t st);
+
 // Per-pass values read from device memory, so that one captured graph serves
 // every pass of the same shape (the host writes them before each replay).
 struct PassParams {
