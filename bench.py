@@ -725,12 +725,14 @@ def record_name(symbol):
         s = s.replace(junk, "")
     m = re.match(r"(k_\w+)<(.*)>$", s)
     if not m:
-        return s
+        return "k_combine_rows<float>" if s == "k_combine_rows" else s
     name, a = m.group(1), m.group(2).split(",")
     if name == "k_sub" and len(a) == 5:
         return "k_sub<" + ",".join(a[:4] + ([] if a[4] == "4" else ["1"])) + ">"
-    if name == "k_hub_seq":
-        return f"k_hub_seq<{a[0]}>"
+    if name in ("k_hub_seq", "k_root_seq"):
+        return f"{name}<{a[0]}>"
+    if name == "k_stream":
+        return "k_stream<float>"
     if name == "k_runs" and len(a) == 5:
         return f"k_runs<{a[0]},{ {'0': 'fwd', '1': 't'}.get(a[3], a[3]) },{a[4]}>"
     if name in ("k_runs_g", "k_runs_tg"):
@@ -739,6 +741,8 @@ def record_name(symbol):
         return f"k_runs<{a[0]},seq,{a[3]}>"
     if name in ("k_bwd_node", "k_bwd_node_lds", "k_bwd_node_rows"):
         return f"k_bwd_node<{a[0]}>"
+    if name == "k_bwd_node_rows16":
+        return "k_bwd_node<float>"
     if name in ("k_edge_grad", "k_fascia_step"):
         return f"{name}<{a[0]}>"
     return s

@@ -1143,7 +1143,8 @@ __global__ __launch_bounds__(256) void k_bwd_node_lds(const NodeArgs<T> a, int v
 // collide once per 16-byte read instead of once per row.  Rows past the
 // group's last are zero-filled and their sums not stored.  Per row the same
 // sum, in the same order, as k_bwd_node_lds.  Steps below the root (a G
-// table) whose Y is not the histogram.
+// table) whose Y is not the histogram: FP64 ones, and FP32 ones whose rows and
+// lists exceed k_bwd_node_rows16's LDS.
 constexpr int kNodeRows = 8;
 
 // R consecutive values of T from 16-byte aligned LDS
@@ -1293,6 +1294,10 @@ hipError_t launch_bwd_node_t(const NodeArgs<T>& a, int num_cus, hipStream_t st)
         hipLaunchKernelGGL((k_bwd_node<T, Acc>), flat_grid(total), dim3(256), 0, st, a);
         return hipGetLastError();
     }
+    if constexpr (sizeof(T) == 4)
+        if (a.rows_inner && a.G && a.Tm && !a.y_from_h && a.Wo < 1024 && a.Wm < 1024 && a.Wy < 1024 &&
+            node_rows16_lds_bytes(a) <= kNodeRows16Lds)
+            return launch_bwd_node_rows16(a, num_cus, st);
     const size_t lists = (size_t)4 * (((do_dy && a.Tm) ? (size_t)a.Pa * a.Wy : 0) + (do_gm ? (size_t)a.Pm * a.Wm : 0));
     const size_t lists_head = (lists + 15) & ~(size_t)15;
     auto vpb_for = [&](size_t budget) {

@@ -287,6 +287,13 @@ struct NodeArgs {
 template <typename T>
 hipError_t launch_bwd_node(const NodeArgs<T>& a, int num_cus, hipStream_t st);
 
+// The same for FP32 steps below the root with a main table and a Y of their
+// own, 16 rows side by side in LDS (pg_combine.hip); up to kNodeRows16Lds bytes
+// of it, two workgroups a CU.
+constexpr size_t kNodeRows16Lds = 80 * 1024 - 64;
+size_t node_rows16_lds_bytes(const NodeArgs<float>& a);
+hipError_t launch_bwd_node_rows16(const NodeArgs<float>& a, int num_cus, hipStream_t st);
+
 // Per entry e = (row v, column u): grad[e] += sum_b sum_i dY[v][b][i] * T_a-term(u)
 // (aux table) or dY[v][b][i(col u)] (aux leaf).  One thread per entry.
 template <typename T>
