@@ -791,6 +791,20 @@ template <typename T>
 int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, int y_cols, StepBytes bytes,
                            bool rows);
 
+// Narrow rows loaded whole and permuted (k_stream) against k_sub's permuted
+// loads: always where the rows are no wider than the sums; where they are
+// wider it loads more than it uses, and gains while it needs few chunks of
+// colorings.  R-MAT scale 18, ms by k_stream / k_sub, rows -> sums: 1
+// coloring 15 -> 20 0.10 / 0.18; 4 colorings 28 -> 8 0.21 / 0.30 (2 chunks),
+// 56 -> 28 0.43 / 0.51 (4), 36 -> 9 0.42 / 0.30 (4); 16 colorings 6 -> 4
+// 0.21 / 0.25 (2), 15 -> 6 0.44 / 0.52 (4), 20 -> 15 0.76 / 0.77 (6), 21 -> 7
+// 0.80 / 0.63 (6), 35 -> 21 1.64 / 1.43 (16), 9 -> 36 1.5 / 1.8.
+bool stream_gains(int B, int Wy, int Wa)
+{
+    const int most = stream_colorings(B, Wy, Wa), chunks = (B + most - 1) / most;
+    return Wa <= Wy || chunks <= 2 || (chunks <= 4 && Wa <= 3 * Wy);
+}
+
 template <typename T>
 int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, int y_cols, StepBytes bytes,
                      int used_per_mille = 0)
@@ -822,11 +836,28 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         if (N > 0) b += bytes.per_vertex * verts / N;
         return b;
     };
+    // Rows no wider than the sums by whole rows (k_stream) where most lanes are
+    // used, ms by k_stream / k_sub: 5-path, R-MAT scale 18, 16 colorings, rows of
+    // 4 into 6 values 0.80 / 1.15, of 1 into 4 0.46 / 0.60; 12-vertex tree, scale
+    // 20, 4 colorings, 11 into 55 4.7 / 6.4; scale 22, one coloring 4.3 / 6.4;
+    // but of 1 into 11 there, 11 lanes, 4.1 / 2.1, of 55 into 11 5.3 / 4.6, and
+    // (scale 18 above) of 6 into 4 0.80 / 0.73.
+    const bool stream = sizeof(T) == 4 && aux == AUX_GATHER_TG && a.gidx && a.out_mode == OUT_Y && a.Wa <= a.Wy &&
+                        stream_fits(c->n_act, a.lda, a.Wy, a.Wa) &&
+                        stream_colorings(a.B, a.Wy, a.Wa) * a.Wy >= 40;
     auto hubs = [&](hipStream_t hs) -> int {
         SubArgs<T> h = a;
         h.out = part;
         h.ldo = y_cols;
         h.out_mode = OUT_PARTIAL;
+        if constexpr (sizeof(T) == 4)
+            if (stream) {
+                record(c, "k_stream<float,tg>", share(c->h_rowptr[c->n_hub], 0), true);
+                HIP_TRY(c, launch_stream(STREAM_TG_HUB, h, c->d_hub_items.as<int4>(), c->n_hub_items, nullptr, c->n_act,
+                                         cus, hs));
+                record(c, "", 0, false);
+                return PG_OK;
+            }
         h.items = c->d_hub_items.as<int4>();
         h.n_items = c->n_hub_items;
         h.item_base = 0;
@@ -837,6 +868,14 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         return PG_OK;
     };
     auto rest = [&](hipStream_t rs) -> int {
+        if constexpr (sizeof(T) == 4)
+            if (stream) {
+                record(c, "k_stream<float,tg>", share((double)c->nnz - c->h_rowptr[c->n_hub], c->n_act - c->n_hub), true);
+                HIP_TRY(c, launch_stream(STREAM_TG, a, c->d_stream_tiles.as<int4>(), c->n_stream_tiles,
+                                         c->d_local.as<uint8_t>(), c->n_act, cus, rs));
+                record(c, "", 0, false);
+                return PG_OK;
+            }
         struct Bucket { int32_t lo, hi; int lanes; };
         const Bucket buckets[3] = {{c->n_hub, c->hi_end, 64}, {c->hi_end, c->mid_end, 16}, {c->mid_end, c->n_act, 8}};
         for (const Bucket& bk : buckets) {
@@ -874,17 +913,6 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
     return PG_OK;
 }
 
-// The forward neighbour sums in the reference's order (CSCGraph.hpp:254-307:
-// every Y value adds its neighbours' values one after another, in ascending
-// column order, starting from zero), so the FP32 sums are the reference's,
-// bit for bit:
-//  - hubs: one partial row per hub, each value one running sum over the whole
-//    neighbour list, by k_hub_seq (the wavefronts of a workgroup share the
-//    list and hand the running sums on);
-//  - the other vertices: a team with the whole neighbour list, one
-//    neighbour group, by whole rows (RUNS_SEQ, when `rows`) or by gathers;
-//  - the finishing launch adds each hub's single partial row to zero and
-//    combines it with the main table.
 // the first streaming tile that starts at vertex v or later, and the last
 // vertex in [v0, v] that starts a tile (v itself where the tiles end)
 int tile_of(const pg_ctx* c, int32_t v)
@@ -910,6 +938,19 @@ int32_t tile_floor(const pg_ctx* c, int32_t v0, int32_t v)
 constexpr int64_t kCombineReuse = 2;
 constexpr int64_t kCombineRowsMin = 1 << 14;
 
+// The forward neighbour sums in the reference's order (CSCGraph.hpp:254-307:
+// every Y value adds its neighbours' values one after another, in ascending
+// column order, starting from zero), so the FP32 sums are the reference's,
+// bit for bit:
+//  - hubs: one partial row per hub, each value one running sum over the whole
+//    neighbour list, by k_hub_seq (the wavefronts of a workgroup share the
+//    list and hand the running sums on);
+//  - the other vertices: a team with the whole neighbour list, one
+//    neighbour group, by whole rows (RUNS_SEQ, when `rows`) or by gathers, or
+//    (narrow rows) a wavefront per tile of vertices (k_stream);
+//  - the finishing launch adds each hub's single partial row to zero and
+//    combines it with the main table (the others' combine is fused with their
+//    gather, or a launch of its own, k_combine_rows).
 template <typename T>
 int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, int y_cols, StepBytes bytes,
                            bool rows)
@@ -939,21 +980,9 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
                   combine_rows_lds_bytes(a.Wy, a.Wm, a.Wo, a.P) <= kLdsLimit &&
                   (int64_t)a.P * a.Wo >= kCombineReuse * (a.Wy + a.Wm + a.Wo);
     const int gather_main = by_rows ? MAIN_LEAF : main_mode;  // the gather's own outputs: Y
-    // Narrow rows loaded whole and permuted (k_stream) against k_sub's permuted
-    // loads: always where the rows are no wider than the sums; where they are
-    // wider it loads more than it uses, and gains while it needs few chunks of
-    // colorings.  R-MAT scale 18, ms by k_stream / k_sub, rows -> sums: 1
-    // coloring 15 -> 20 0.10 / 0.18; 4 colorings 28 -> 8 0.21 / 0.30 (2 chunks),
-    // 56 -> 28 0.43 / 0.51 (4), 36 -> 9 0.42 / 0.30 (4); 16 colorings 6 -> 4
-    // 0.21 / 0.25 (2), 15 -> 6 0.44 / 0.52 (4), 20 -> 15 0.76 / 0.77 (6), 21 -> 7
-    // 0.80 / 0.63 (6), 35 -> 21 1.64 / 1.43 (16), 9 -> 36 1.5 / 1.8.
-    bool stream = false;
-    if constexpr (sizeof(T) == 4)
-        if (!rows && gather_main == MAIN_LEAF && (a.out_mode == OUT_EMA || a.out_mode == OUT_EMA_SCALED) && a.gidx &&
-            a.Wy <= 64 && a.Wa <= 63 && (int64_t)c->n_act * a.lda * 4 < ((int64_t)1 << 32) - 16) {
-            const int chunks = (a.B + stream_colorings(a) - 1) / stream_colorings(a);
-            stream = a.Wa <= a.Wy || chunks <= 2 || (chunks <= 4 && a.Wa <= 3 * a.Wy);
-        }
+    const bool stream = sizeof(T) == 4 && !rows && gather_main == MAIN_LEAF &&
+                        (a.out_mode == OUT_EMA || a.out_mode == OUT_EMA_SCALED) && a.gidx &&
+                        stream_fits(c->n_act, a.lda, a.Wy, a.Wa) && stream_gains(a.B, a.Wy, a.Wa);
     a.ng = 1;
     auto hubs = [&](hipStream_t hs) -> int {
         SubArgs<T> h = a;
@@ -979,8 +1008,8 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
             if constexpr (sizeof(T) == 4) {
                 const int t0 = tile_of(c, v0), t1 = tile_of(c, v1);
                 record(c, "k_stream<float>", sh, true);
-                HIP_TRY(c, launch_stream(r, c->d_stream_tiles.as<int4>() + t0, t1 - t0, c->d_local.as<uint8_t>(),
-                                         c->n_act, cus, rs));
+                HIP_TRY(c, launch_stream(STREAM_FORWARD, r, c->d_stream_tiles.as<int4>() + t0, t1 - t0,
+                                         c->d_local.as<uint8_t>(), c->n_act, cus, rs));
             }
         } else if (root_tiles) {
             record(c, sizeof(T) == 4 ? "k_root_seq<float>" : "k_root_seq<double>", sh, true);

@@ -38,16 +38,60 @@ constexpr int kStreamColors = 32;      // colorings of a wavefront at most
 constexpr int kStreamColorBytes = 68;  // LDS bytes per coloring of a batch's colour pairs: an odd number of words
 constexpr int kStreamRowLanes = 63;    // row values a wavefront loads at once; its last lane holds zero
 constexpr int kXcds = 8;
+constexpr int kStreamBatch = 48;       // rows in flight
 constexpr uint32_t kStreamNoValue = 0xfffffff0u;  // a byte offset past every table: the load gives zero
 
 __host__ __device__ constexpr size_t stream_tab_bytes(int k, int Wy) { return ((size_t)(k * k + 1) * Wy + 15) & ~(size_t)15; }
 
-template <int NB>
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+
+// a's sums over lanes l and l ^ BIT (32 or 16) in the lanes without that bit,
+// b's in those with it
+template <int BIT>
+__device__ __forceinline__ float swap_add(float a, float b)
+{
+    const auto r = BIT == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                             : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// The sums over all 64 lanes of 16 values at once: lane l's result is the sum of
+// value l / 4.  Each step adds two lanes and halves the values a lane carries
+// (row rotation by 8, mirror of 8 lanes), then the quad's lanes.
+__device__ __forceinline__ float lane_sums(const float (&p)[16], int lane)
+{
+    float h[8], q[4], r[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) h[i] = swap_add<32>(p[i], p[i + 8]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = swap_add<16>(h[i], h[i + 4]);
+    const bool b3 = lane & 8, b2 = lane & 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) r[i] = (b3 ? q[i + 2] : q[i]) + dpp<0x128>(b3 ? q[i] : q[i + 2]);
+    float x = (b2 ? r[1] : r[0]) + dpp<0x141>(b2 ? r[0] : r[1]);
+    x = x + dpp<0x4e>(x);
+    return x + dpp<0xb1>(x);
+}
+
+// TG: the adjoint's transposed gather, which also takes the gradient of each
+// entry's transpose, the dot of what the entry adds with the vertex's own row:
+// grad[e] += sum over lanes of dy[v] * x, for 16 entries at a time by adds that
+// leave each entry's sum in four lanes (lane_sums; a reduction of its own per
+// entry would take six).  HUB: tiles are {vertex, first entry, end entry,
+// output row}, parts of one list each.
+template <int NB, bool TG, bool HUB>
 __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const int4* tiles, int n_tiles,
                                                    const uint8_t* local, int CB, int nch, uint32_t table_bytes)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    static_assert(NB <= 64, "a batch's entries sit one per lane");
+    constexpr int GR = TG ? 16 : 8;  // entries whose values are brought to their lanes together
+    constexpr int SHARE = 64 / GR;   // lanes that hold the same entry's lane_sums
+    static_assert(NB <= 64 && NB % GR == 0, "a batch's entries sit one per lane");
+    static_assert(NB / GR <= SHARE, "a lane keeps one of its groups' sums");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int B = a.B, Wy = a.Wy, k = a.k;
@@ -70,150 +114,179 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
     // a tile's chunks of colorings go to one XCD (workgroups are dealt to the 8
     // in turn), close in time: they share the lines of the neighbour colours
     // and those where two segments of a row meet
-    const int64_t n_work = (int64_t)((n_tiles + kXcds - 1) / kXcds) * nch;
+    // (TG: in one wavefront, one after another, so that an entry's gradient adds
+    // its chunks in a fixed order)
+    const int apart = TG ? 1 : nch;
+    const int64_t n_work = (int64_t)((n_tiles + kXcds - 1) / kXcds) * apart;
     const int64_t step = (int64_t)(gridDim.x / kXcds) * (kBlock / 64);
     for (int64_t work = (int64_t)(blockIdx.x / kXcds) * (kBlock / 64) + wave; work < n_work; work += step) {
-        const int tile = (int)(work / nch) * kXcds + (int)(blockIdx.x % kXcds);
-        const int b0 = (int)(work % nch) * CB;
+        const int tile = (int)(work / apart) * kXcds + (int)(blockIdx.x % kXcds);
+        const int b_first = (int)(work % apart) * CB;
         if (tile >= n_tiles) continue;
-        const int nc = min(CB, B - b0);
-        const int4 t4 = tiles[tile];  // first vertex, vertices, first entry, entries
-        const int v0 = t4.x, e0 = t4.z, e1 = t4.z + t4.w;
-        const bool mine = lane < nc * Wy;
-        const int c = min(lane_coloring, nc - 1);
-        const int shift = c * a.Wa * 4;
-        const uint32_t place = lane < nc * a.Wa ? (uint32_t)(b0 * a.Wa + lane) * 4u : kStreamNoValue;
-        const int nbat = (t4.w + NB - 1) / NB;
-        // lane j < NB holds entry j of a batch; one past the tile reads its
-        // first entry with colours that add nothing
-        int um = 0, lv = 0, lv_next = 0;
-        float wm = 1.0f;
-        bool last = false;
-        uint32_t pd[kStreamColors / 4];
-        uint32_t pt[3];
-        auto locate = [&](int t) {
-            const int e = e0 + t * NB + lane;
-            const int ec = e < e1 ? e : e0;
-            lv = local[ec];
-            lv_next = e + 1 < e1 ? (int)local[ec + 1] : -1;
-        };
-        auto meta = [&](int t) {  // after locate(t)
-            const int e = e0 + t * NB + lane;
-            const bool ok = lane < NB && e < e1;
-            const int ec = ok ? e : e0;
-            last = ok && lv_next != lv;
-            um = (int)((uint32_t)a.col[ec] * rowbytes);
-            wm = a.w && ok ? a.w[ec] : 1.0f;
-            const uint8_t* ep = a.ecol + (int64_t)ec * B + b0;
-            const uint8_t* vp = a.colors + (int64_t)(v0 + lv) * B + b0;
-            const uint32_t none = (uint32_t)(k * k);
+        int b0 = b_first;
+        do {
+            const int nc = min(CB, B - b0);
+            const int4 t4 = tiles[tile];  // first vertex, vertices, first entry, entries
+            const int v0 = t4.x, e0 = HUB ? t4.y : t4.z, e1 = HUB ? t4.z : t4.z + t4.w;
+            const int v_last = HUB ? v0 : v0 + t4.y - 1;
+            const bool mine = lane < nc * Wy;
+            const int c = min(lane_coloring, nc - 1);
+            const int shift = TG && !mine ? kStreamRowLanes * 4 : c * a.Wa * 4;  // (past the values: none)
+            const uint32_t place = lane < nc * a.Wa ? (uint32_t)(b0 * a.Wa + lane) * 4u : kStreamNoValue;
+            const int nbat = (e1 - e0 + NB - 1) / NB;
+            // lane j < NB holds entry j of a batch; one past the tile reads its
+            // first entry with colours that add nothing
+            int um = 0, lv = 0, lv_next = 0;
+            float wm = 1.0f;
+            bool last = false;
+            uint32_t pd[kStreamColors / 4];
+            uint32_t pt[3];
+            auto locate = [&](int t) {
+                if (HUB) return;
+                const int e = e0 + t * NB + lane;
+                const int ec = e < e1 ? e : e0;
+                lv = local[ec];
+                lv_next = e + 1 < e1 ? (int)local[ec + 1] : -1;
+            };
+            auto meta = [&](int t) {  // after locate(t)
+                const int e = e0 + t * NB + lane;
+                const bool ok = lane < NB && e < e1;
+                const int ec = ok ? e : e0;
+                last = ok && (HUB ? e + 1 == e1 : lv_next != lv);
+                um = (int)((uint32_t)a.col[ec] * rowbytes);
+                wm = a.w && ok ? a.w[ec] : 1.0f;
+                const uint8_t* ep = a.ecol + (int64_t)ec * B + b0;
+                const uint8_t* vp = a.colors + (int64_t)(v0 + lv) * B + b0;
+                const uint32_t none = (uint32_t)(k * k);
 #pragma unroll
-            for (int d = 0; d < kStreamColors / 4; ++d)
-                if (4 * d + 4 <= nc) {
-                    uint32_t x, y;
-                    __builtin_memcpy(&x, ep + 4 * d, 4);
-                    __builtin_memcpy(&y, vp + 4 * d, 4);
-                    // four colour pairs at once: cv * k + cu < 256 carries into no neighbour
-                    pd[d] = ok ? y * (uint32_t)k + x : none * 0x01010101u;
-                }
+                for (int d = 0; d < kStreamColors / 4; ++d)
+                    if (4 * d + 4 <= nc) {
+                        uint32_t x, y;
+                        __builtin_memcpy(&x, ep + 4 * d, 4);
+                        __builtin_memcpy(&y, vp + 4 * d, 4);
+                        // four colour pairs at once: cv * k + cu < 256 carries into no neighbour
+                        pd[d] = ok ? y * (uint32_t)k + x : none * 0x01010101u;
+                    }
 #pragma unroll
-            for (int r = 0; r < 3; ++r)
-                if (r < (nc & 3)) pt[r] = ok ? (uint32_t)vp[(nc & ~3) + r] * (uint32_t)k + ep[(nc & ~3) + r] : none;
-        };
-        locate(0);
-        meta(0);
-        if (nbat > 1) locate(1);
-        float acc = 0.0f;
-        int v = v0;
-        for (int t = 0; t < nbat; ++t) {
-            const int uc = um;
-            const float wc = wm;
-            const uint64_t ends = __ballot(last);
-            unsigned char* to = s_pair + lane;
-#pragma unroll
-            for (int d = 0; d < kStreamColors / 4; ++d)
-                if (4 * d + 4 <= nc)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) to[(4 * d + r) * kStreamColorBytes] = (unsigned char)(pd[d] >> (8 * r));
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-                if (r < (nc & 3)) to[((nc & ~3) + r) * kStreamColorBytes] = (unsigned char)pt[r];
-            wave_sync();
-            float x[NB];
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-                x[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    table, (int)place, __builtin_amdgcn_readlane(uc, j), 0));
-            if (t + 1 < nbat) {
-                meta(t + 1);  // the next batch's ids, behind this one's rows
-                if (t + 2 < nbat) locate(t + 2);
+                for (int r = 0; r < 3; ++r)
+                    if (r < (nc & 3)) pt[r] = ok ? (uint32_t)vp[(nc & ~3) + r] * (uint32_t)k + ep[(nc & ~3) + r] : none;
+            };
+            locate(0);
+            meta(0);
+            if (nbat > 1) locate(1);
+            float acc = 0.0f;
+            int v = v0;
+            // TG: the lane's values of the own rows of v and of the vertex after it
+            auto own_row = [&](int u) {
+                return mine ? a.dy[(int64_t)min(u, v_last) * a.ldd + b0 * Wy + lane] : 0.0f;
+            };
+            float own = 0.0f, own_next = 0.0f;
+            if (TG) {
+                own = own_row(v0);
+                own_next = own_row(v0 + 1);
             }
-            const unsigned char* from = s_pair + c * kStreamColorBytes;
-            // the lanes' values first, a group at a time, without a branch
-            // between them: their LDS reads and permutes overlap
-            constexpr int GR = 8;
+            for (int t = 0; t < nbat; ++t) {
+                const int uc = um;
+                const float wc = wm;
+                const uint64_t ends = __ballot(last);
+                unsigned char* to = s_pair + lane;
 #pragma unroll
-            for (int g = 0; g < NB; g += GR) {
-                int at[GR];
+                for (int d = 0; d < kStreamColors / 4; ++d)
+                    if (4 * d + 4 <= nc)
 #pragma unroll
-                for (int j = 0; j < GR; j += 4) {
-                    const uint32_t p4 = *reinterpret_cast<const uint32_t*>(from + g + j);
+                        for (int r = 0; r < 4; ++r) to[(4 * d + r) * kStreamColorBytes] = (unsigned char)(pd[d] >> (8 * r));
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) at[j + r] = (int)((p4 >> (8 * r)) & 255u);
+                for (int r = 0; r < 3; ++r)
+                    if (r < (nc & 3)) to[((nc & ~3) + r) * kStreamColorBytes] = (unsigned char)pt[r];
+                wave_sync();
+                float x[NB];
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    x[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        table, (int)place, __builtin_amdgcn_readlane(uc, j), 0));
+                if (t + 1 < nbat) {
+                    meta(t + 1);  // the next batch's ids, behind this one's rows
+                    if (t + 2 < nbat) locate(t + 2);
                 }
+                const unsigned char* from = s_pair + c * kStreamColorBytes;
+                float sums = 0.0f;
+                // the lanes' values first, a group at a time, without a branch
+                // between them: their LDS reads and permutes overlap
 #pragma unroll
-                for (int j = 0; j < GR; ++j) at[j] = min((int)tab[__umul24((uint32_t)at[j], (uint32_t)Wy)] + shift, kStreamRowLanes * 4);
+                for (int g = 0; g < NB; g += GR) {
+                    int at[GR];
 #pragma unroll
-                for (int j = 0; j < GR; ++j)
-                    x[g + j] = __int_as_float(__builtin_amdgcn_ds_bpermute(at[j], __float_as_int(x[g + j])));
-                if (a.w)
+                    for (int j = 0; j < GR; j += 4) {
+                        const uint32_t p4 = *reinterpret_cast<const uint32_t*>(from + g + j);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) at[j + r] = (int)((p4 >> (8 * r)) & 255u);
+                    }
 #pragma unroll
                     for (int j = 0; j < GR; ++j)
-                        x[g + j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wc), g + j)) * x[g + j];
-                const uint32_t e8 = (uint32_t)(ends >> g) & ((1u << GR) - 1u);
-                if (e8 == 0) {
+                        at[j] = min((int)tab[__umul24((uint32_t)at[j], (uint32_t)Wy)] + shift, kStreamRowLanes * 4);
 #pragma unroll
-                    for (int j = 0; j < GR; ++j) acc = acc + x[g + j];
-                } else {
+                    for (int j = 0; j < GR; ++j)
+                        x[g + j] = __int_as_float(__builtin_amdgcn_ds_bpermute(at[j], __float_as_int(x[g + j])));
+                    float p[GR];  // TG: of the values without their weights
+                    if (!TG && a.w)
 #pragma unroll
-                    for (int j = 0; j < GR; ++j) {
-                        acc = acc + x[g + j];
-                        if ((e8 >> j) & 1) {
-                            if (mine) {
-                                const float out =
-                                    a.out_mode == OUT_EMA_SCALED ? (float)((double)acc * (double)a.scale) : acc;
-                                a.out[(int64_t)v * a.ldo + b0 * Wy + lane] = out;
-                                if (a.ykeep) a.ykeep[(int64_t)v * a.ldy + b0 * Wy + lane] = acc;
+                        for (int j = 0; j < GR; ++j)
+                            x[g + j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wc), g + j)) * x[g + j];
+                    auto scaled = [&](int j) {
+                        if (!TG || !a.w) return x[g + j];
+                        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wc), g + j)) * x[g + j];
+                    };
+                    const uint32_t group_ends = (uint32_t)(ends >> g) & ((1u << GR) - 1u);
+                    if (group_ends == 0) {
+#pragma unroll
+                        for (int j = 0; j < GR; ++j) acc = acc + scaled(j);
+                        if (TG)
+#pragma unroll
+                            for (int j = 0; j < GR; ++j) p[j] = own * x[g + j];
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < GR; ++j) {
+                            acc = acc + scaled(j);
+                            if (TG) p[j] = own * x[g + j];
+                            if ((group_ends >> j) & 1) {
+                                if (mine) {
+                                    float out = acc;
+                                    if (!TG && a.out_mode == OUT_EMA_SCALED) out = (float)((double)acc * (double)a.scale);
+                                    const int64_t row = HUB ? t4.w : v;
+                                    a.out[row * a.ldo + b0 * Wy + lane] = out;
+                                    if (!TG && a.ykeep) a.ykeep[(int64_t)v * a.ldy + b0 * Wy + lane] = acc;
+                                }
+                                acc = 0.0f;
+                                ++v;
+                                if (TG && !HUB) {
+                                    own = own_next;
+                                    own_next = own_row(v + 1);
+                                }
                             }
-                            acc = 0.0f;
-                            ++v;
                         }
                     }
+                    if constexpr (TG) {
+                        const float s = lane_sums(p, lane);
+                        if (lane % SHARE == g / GR) sums = s;
+                    }
                 }
+                if constexpr (TG) {
+                    const int j = lane % SHARE * GR + lane / SHARE;
+                    const int e = e0 + t * NB + j;
+                    if (j < NB && e < e1) (void)unsafeAtomicAdd(&a.grad[e], (double)sums);  // (returns nothing: no wait)
+                }
+                wave_sync();  // the pairs are read before the next batch's are written
             }
-            wave_sync();  // the pairs are read before the next batch's are written
-        }
+            b0 += CB;
+        } while (TG && b0 < B);
     }
 }
 
-constexpr int kStreamBatch = 48;
-
-}  // namespace
-
-int stream_colorings(const SubArgs<float>& a)
+template <bool TG, bool HUB>
+hipError_t launch_stream_t(const SubArgs<float>& a, const int4* tiles, int n_tiles, const uint8_t* local,
+                           uint32_t table_bytes, int num_cus, hipStream_t st)
 {
-    return std::min({a.B, 64 / a.Wy, kStreamRowLanes / a.Wa, kStreamColors});
-}
-
-hipError_t launch_stream(const SubArgs<float>& a, const int4* tiles, int n_tiles, const uint8_t* local, int64_t n_rows,
-                         int num_cus, hipStream_t st)
-{
-    if (n_tiles <= 0) return hipSuccess;
-    const int64_t table_bytes = n_rows * a.lda * 4;
-    if (a.out_mode != OUT_EMA && a.out_mode != OUT_EMA_SCALED) return hipErrorInvalidValue;
-    if (a.Wy > 64 || a.Wa > kStreamRowLanes || a.k > kMaxK || !a.gidx || table_bytes > (int64_t)kStreamNoValue)
-        return hipErrorInvalidValue;
-    const int most = stream_colorings(a);
+    const int most = stream_colorings(a.B, a.Wy, a.Wa);
     const int nch = (a.B + most - 1) / most;
     const int CB = (a.B + nch - 1) / nch;
     const size_t lds = stream_tab_bytes(a.k, a.Wy) + (size_t)(kBlock / 64) * kStreamColors * kStreamColorBytes;
@@ -221,17 +294,44 @@ hipError_t launch_stream(const SubArgs<float>& a, const int4* tiles, int n_tiles
     auto it = per_cu_cache.find(lds);
     if (it == per_cu_cache.end()) {
         int per_cu = 0;
-        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stream<kStreamBatch>, kBlock, lds);
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stream<kStreamBatch, TG, HUB>, kBlock, lds);
         if (e != hipSuccess) return e;
         if (per_cu < 1) return hipErrorInvalidConfiguration;
         it = per_cu_cache.emplace(lds, per_cu).first;
     }
-    const int64_t need = ((int64_t)n_tiles * nch + kBlock / 64 - 1) / (kBlock / 64);
+    const int64_t need = ((int64_t)n_tiles * (TG ? 1 : nch) + kBlock / 64 - 1) / (kBlock / 64);
     const int64_t most_blocks = std::min<int64_t>(need, (int64_t)it->second * num_cus);
     const int grid = (int)((most_blocks + kXcds - 1) / kXcds) * kXcds;
-    hipLaunchKernelGGL((k_stream<kStreamBatch>), dim3(grid), dim3(kBlock), lds, st, a, tiles, n_tiles, local, CB, nch,
-                       (uint32_t)table_bytes);
+    hipLaunchKernelGGL((k_stream<kStreamBatch, TG, HUB>), dim3(grid), dim3(kBlock), lds, st, a, tiles, n_tiles, local, CB, nch,
+                       table_bytes);
     return hipGetLastError();
+}
+
+}  // namespace
+
+int stream_colorings(int B, int Wy, int Wa)
+{
+    return std::min({B, 64 / Wy, kStreamRowLanes / Wa, kStreamColors});
+}
+
+bool stream_fits(int64_t n_rows, int lda, int Wy, int Wa)
+{
+    return Wy >= 1 && Wy <= 64 && Wa >= 1 && Wa <= kStreamRowLanes && n_rows * lda * 4 <= (int64_t)kStreamNoValue;
+}
+
+hipError_t launch_stream(StreamMode mode, const SubArgs<float>& a, const int4* tiles, int n_tiles,
+                         const uint8_t* local, int64_t n_rows, int num_cus, hipStream_t st)
+{
+    if (n_tiles <= 0) return hipSuccess;
+    if (a.k > kMaxK || !a.gidx || !stream_fits(n_rows, a.lda, a.Wy, a.Wa)) return hipErrorInvalidValue;
+    const uint32_t bytes = (uint32_t)(n_rows * a.lda * 4);
+    if (mode == STREAM_FORWARD) {
+        if (a.out_mode != OUT_EMA && a.out_mode != OUT_EMA_SCALED) return hipErrorInvalidValue;
+        return launch_stream_t<false, false>(a, tiles, n_tiles, local, bytes, num_cus, st);
+    }
+    if (!a.dy || !a.grad || (a.out_mode != OUT_Y && a.out_mode != OUT_PARTIAL)) return hipErrorInvalidValue;
+    return mode == STREAM_TG ? launch_stream_t<true, false>(a, tiles, n_tiles, local, bytes, num_cus, st)
+                             : launch_stream_t<true, true>(a, tiles, n_tiles, local, bytes, num_cus, st);
 }
 
 __global__ void k_local_ids(uint8_t* local, const int4* tiles, int n_tiles, const int32_t* rowptr)

@@ -78,3 +78,33 @@ def test_streamed_rows_keep_the_reference_arithmetic(gpu_ctx, k, edges, coloring
         gpu_ctx.set_weights(None)
         for key, v in zip(keys, saved):
             gpu_ctx.set_option(key, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hub_degree", [64, 4096])
+@pytest.mark.parametrize("k,edges,colorings", [
+    (5, U5, (12, 33)),       # rows of 4 into 6 values and of 1 into 4, two and more chunks
+    (12, PATH12, (1, 4)),    # rows of 11 into 55, a coloring a chunk
+])
+def test_streamed_gradients_of_every_entry(gpu_ctx, k, edges, colorings, hub_degree):
+    """FP32 gradients of weighted counts equal the FP64 ones, entry by entry, up
+    to FP32 rounding: of at most 1,500 products and additions a step forward and
+    as many backward, all non-negative."""
+    n, colptr, rowidx = _graph()
+    saved = gpu_ctx.get_option("hub_degree")
+    try:
+        gpu_ctx.set_option("hub_degree", hub_degree)
+        gpu_ctx.upload_graph(colptr, rowidx)
+        rng = np.random.default_rng(71 + k)
+        gpu_ctx.set_weights(rng.uniform(0.5, 1.5, len(rowidx)).astype(np.float32))
+        plan = gpu_ctx.plan(k, edges)
+        tol = 2 * (k - 1) * 1510 * 2.0**-24
+        for B in colorings:
+            cols = rng.integers(0, k, size=(B, n)).astype(np.uint8)
+            print(f"[stream grad] k={k} B={B} hub_degree={hub_degree}", flush=True)
+            _, g32 = gpu_ctx.count_grad(plan, B, colors=cols, precision="fp32")
+            _, g64 = gpu_ctx.count_grad(plan, B, colors=cols, precision="fp64")
+            assert np.all(np.abs(g32 - g64) <= tol * np.abs(g64)), np.abs(g32 / g64 - 1)[g64 > 0].max()
+    finally:
+        gpu_ctx.set_weights(None)
+        gpu_ctx.set_option("hub_degree", saved)
