@@ -732,7 +732,7 @@ def record_name(symbol):
     if name in ("k_hub_seq", "k_root_seq"):
         return f"{name}<{a[0]}>"
     if name == "k_stream":
-        return "k_stream<float,tg>" if a[1:2] == ["true"] else "k_stream<float>"
+        return f"k_stream<{a[0]},tg>" if a[2:3] == ["true"] else f"k_stream<{a[0]}>"
     if name == "k_runs" and len(a) == 5:
         return f"k_runs<{a[0]},{ {'0': 'fwd', '1': 't'}.get(a[3], a[3]) },{a[4]}>"
     if name in ("k_runs_g", "k_runs_tg"):

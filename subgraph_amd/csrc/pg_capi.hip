@@ -805,6 +805,20 @@ bool stream_gains(int B, int Wy, int Wa)
     return Wa <= Wy || chunks <= 2 || (chunks <= 4 && Wa <= 3 * Wy);
 }
 
+// FP64 rows are twice as long for the same values, so the streamed sums gain
+// less: where half of the lanes are used, the rows are no wider than the sums,
+// and the hubs hold a quarter of the entries, so that most rows read lie in the
+// L2 (a graph without hubs is bound by the memory behind it, by k_sub as well).
+// Calls, ms by k_sub / with this: 7-vertex tree, R-MAT scale 20, 16 colorings
+// 15.1 / 13.3; 10-vertex, scale 18, 4 colorings 10.4 / 10.2; 5-path, scale 18,
+// 16 colorings 2.20 / 2.13.  Outside the rule: 7-vertex tree, scale 20, one
+// coloring, 20 lanes 1.64 / 1.79; uniform graph, 3 colorings 1.46 / 1.49; the
+// 5-path there, 16 colorings 2.55 / 2.59.
+bool stream_gains_fp64(const pg_ctx* c, int B, int Wy, int Wa)
+{
+    return Wa <= Wy && stream_colorings(B, Wy, Wa) * Wy >= 32 && c->h_rowptr[c->n_hub] >= c->nnz / 4;
+}
+
 template <typename T>
 int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, int y_cols, StepBytes bytes,
                      int used_per_mille = 0)
@@ -843,7 +857,7 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
     // but of 1 into 11 there, 11 lanes, 4.1 / 2.1, of 55 into 11 5.3 / 4.6, and
     // (scale 18 above) of 6 into 4 0.80 / 0.73.
     const bool stream = sizeof(T) == 4 && aux == AUX_GATHER_TG && a.gidx && a.out_mode == OUT_Y && a.Wa <= a.Wy &&
-                        stream_fits(c->n_act, a.lda, a.Wy, a.Wa) &&
+                        stream_fits(c->n_act, (int64_t)a.lda * sizeof(T), a.Wy, a.Wa) &&
                         stream_colorings(a.B, a.Wy, a.Wa) * a.Wy >= 40;
     auto hubs = [&](hipStream_t hs) -> int {
         SubArgs<T> h = a;
@@ -853,8 +867,8 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         if constexpr (sizeof(T) == 4)
             if (stream) {
                 record(c, "k_stream<float,tg>", share(c->h_rowptr[c->n_hub], 0), true);
-                HIP_TRY(c, launch_stream(STREAM_TG_HUB, h, c->d_hub_items.as<int4>(), c->n_hub_items, nullptr, c->n_act,
-                                         cus, hs));
+                HIP_TRY(c, launch_stream<T>(STREAM_TG_HUB, h, c->d_hub_items.as<int4>(), c->n_hub_items, nullptr, c->n_act,
+                                            cus, hs));
                 record(c, "", 0, false);
                 return PG_OK;
             }
@@ -871,8 +885,8 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         if constexpr (sizeof(T) == 4)
             if (stream) {
                 record(c, "k_stream<float,tg>", share((double)c->nnz - c->h_rowptr[c->n_hub], c->n_act - c->n_hub), true);
-                HIP_TRY(c, launch_stream(STREAM_TG, a, c->d_stream_tiles.as<int4>(), c->n_stream_tiles,
-                                         c->d_local.as<uint8_t>(), c->n_act, cus, rs));
+                HIP_TRY(c, launch_stream<T>(STREAM_TG, a, c->d_stream_tiles.as<int4>(), c->n_stream_tiles,
+                                            c->d_local.as<uint8_t>(), c->n_act, cus, rs));
                 record(c, "", 0, false);
                 return PG_OK;
             }
@@ -980,9 +994,10 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
                   combine_rows_lds_bytes(a.Wy, a.Wm, a.Wo, a.P) <= kLdsLimit &&
                   (int64_t)a.P * a.Wo >= kCombineReuse * (a.Wy + a.Wm + a.Wo);
     const int gather_main = by_rows ? MAIN_LEAF : main_mode;  // the gather's own outputs: Y
-    const bool stream = sizeof(T) == 4 && !rows && gather_main == MAIN_LEAF &&
+    const bool stream = !rows && gather_main == MAIN_LEAF &&
                         (a.out_mode == OUT_EMA || a.out_mode == OUT_EMA_SCALED) && a.gidx &&
-                        stream_fits(c->n_act, a.lda, a.Wy, a.Wa) && stream_gains(a.B, a.Wy, a.Wa);
+                        stream_fits(c->n_act, (int64_t)a.lda * sizeof(T), a.Wy, a.Wa) &&
+                        (sizeof(T) == 4 ? stream_gains(a.B, a.Wy, a.Wa) : stream_gains_fp64(c, a.B, a.Wy, a.Wa));
     a.ng = 1;
     auto hubs = [&](hipStream_t hs) -> int {
         SubArgs<T> h = a;
@@ -1005,12 +1020,10 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         r.n_items = v1 - v0;
         const double sh = share((double)c->h_rowptr[v1] - c->h_rowptr[v0], by_rows && mm != main_mode ? 0 : v1 - v0);
         if (streamed) {
-            if constexpr (sizeof(T) == 4) {
-                const int t0 = tile_of(c, v0), t1 = tile_of(c, v1);
-                record(c, "k_stream<float>", sh, true);
-                HIP_TRY(c, launch_stream(STREAM_FORWARD, r, c->d_stream_tiles.as<int4>() + t0, t1 - t0,
-                                         c->d_local.as<uint8_t>(), c->n_act, cus, rs));
-            }
+            const int t0 = tile_of(c, v0), t1 = tile_of(c, v1);
+            record(c, sizeof(T) == 4 ? "k_stream<float>" : "k_stream<double>", sh, true);
+            HIP_TRY(c, launch_stream<T>(STREAM_FORWARD, r, c->d_stream_tiles.as<int4>() + t0, t1 - t0,
+                                        c->d_local.as<uint8_t>(), c->n_act, cus, rs));
         } else if (root_tiles) {
             record(c, sizeof(T) == 4 ? "k_root_seq<float>" : "k_root_seq<double>", sh, true);
             HIP_TRY(c, launch_root_seq<T>(r, c->d_root_tiles.as<int4>(), c->n_root_tiles, cus, rs));

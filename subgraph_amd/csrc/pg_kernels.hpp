@@ -214,7 +214,7 @@ constexpr int kRootTileEntries = 1024, kRootTileVertices = kBlock;
 template <typename T>
 hipError_t launch_root_seq(const SubArgs<T>& a, const int4* tiles, int n_tiles, int num_cus, hipStream_t st);
 
-// Sums of narrow FP32 rows, loaded whole, for tiles of vertices (pg_stream.hip).
+// Sums of narrow rows, loaded whole, for tiles of vertices (pg_stream.hip).
 // Tiles {first vertex, vertices, first entry, entries} of up to
 // kStreamTileVertices vertices; local[e]: the place of entry e's vertex in its
 // tile.  n_rows: rows of the gathered table (of less than 4 GB).
@@ -225,9 +225,10 @@ enum StreamMode : int {
     STREAM_TG_HUB = 2,   // GATHER_TG of work items {vertex, first entry, end entry, slot}, OUT_PARTIAL
 };
 int stream_colorings(int B, int Wy, int Wa);  // colorings a wavefront takes together
-bool stream_fits(int64_t n_rows, int lda, int Wy, int Wa);
-hipError_t launch_stream(StreamMode mode, const SubArgs<float>& a, const int4* tiles, int n_tiles,
-                         const uint8_t* local, int64_t n_rows, int num_cus, hipStream_t st);
+bool stream_fits(int64_t n_rows, int64_t row_bytes, int Wy, int Wa);
+template <typename T>
+hipError_t launch_stream(StreamMode mode, const SubArgs<T>& a, const int4* tiles, int n_tiles, const uint8_t* local,
+                         int64_t n_rows, int num_cus, hipStream_t st);
 hipError_t launch_local_ids(uint8_t* local, const int4* tiles, int n_tiles, const int32_t* rowptr, hipStream_t st);
 
 // The combine of n FP32 rows whose Y is in memory (pg_combine.hip): dense rows

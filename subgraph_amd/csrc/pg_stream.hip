@@ -25,6 +25,10 @@
 // The others wait on latency and lane work: batches of 32 entries, which give
 // more wavefronts, take 1-12% longer, of 56 the same; the values of a vertex
 // added one by one under a branch instead of eight at a time, 5-30% longer.
+// FP64, batches of 32: 7-vertex tree, scale 20, 16 colorings 15.1 -> 13.3 ms a
+// call; 10-vertex, scale 18, 4 colorings 10.4 -> 10.2.  Its transposed gather
+// with gradients stays with k_sub: 158-190 VGPRs here, 5-path, scale 18, 16
+// colorings 5.39 ms a call by k_sub, 5.67 by this kernel.
 #include "pg_kernels.hpp"
 
 #include <algorithm>
@@ -38,15 +42,60 @@ constexpr int kStreamColors = 32;      // colorings of a wavefront at most
 constexpr int kStreamColorBytes = 68;  // LDS bytes per coloring of a batch's colour pairs: an odd number of words
 constexpr int kStreamRowLanes = 63;    // row values a wavefront loads at once; its last lane holds zero
 constexpr int kXcds = 8;
-constexpr int kStreamBatch = 48;       // rows in flight
+// rows in flight
+template <typename T>
+constexpr int kStreamBatch = sizeof(T) == 4 ? 48 : 32;
 constexpr uint32_t kStreamNoValue = 0xfffffff0u;  // a byte offset past every table: the load gives zero
 
 __host__ __device__ constexpr size_t stream_tab_bytes(int k, int Wy) { return ((size_t)(k * k + 1) * Wy + 15) & ~(size_t)15; }
+
+// 64-bit values by their two halves
+__device__ __forceinline__ double join(uint32_t lo, uint32_t hi)
+{
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ uint32_t low(double x) { return (uint32_t)__double_as_longlong(x); }
+__device__ __forceinline__ uint32_t high(double x) { return (uint32_t)((uint64_t)__double_as_longlong(x) >> 32); }
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x)
 {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ float lane_value(float x, int j)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j));
+}
+
+__device__ __forceinline__ double lane_value(double x, int j)
+{
+    return join((uint32_t)__builtin_amdgcn_readlane((int)low(x), j), (uint32_t)__builtin_amdgcn_readlane((int)high(x), j));
+}
+
+// the value of lane at / 4
+__device__ __forceinline__ float permuted(int at, float x)
+{
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(at, __float_as_int(x)));
+}
+
+__device__ __forceinline__ double permuted(int at, double x)
+{
+    return join((uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)low(x)),
+                (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)high(x)));
+}
+
+// the value at byte off + row of the table, zero past its end
+template <typename T>
+__device__ __forceinline__ T table_value(__amdgpu_buffer_rsrc_t table, uint32_t off, int row)
+{
+    if constexpr (sizeof(T) == 4) {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(table, (int)off, row, 0));
+    } else {
+        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(table, (int)off, row, 0);
+        return join(v.x, v.y);
+    }
 }
 
 // a's sums over lanes l and l ^ BIT (32 or 16) in the lanes without that bit,
@@ -83,8 +132,8 @@ __device__ __forceinline__ float lane_sums(const float (&p)[16], int lane)
 // leave each entry's sum in four lanes (lane_sums; a reduction of its own per
 // entry would take six).  HUB: tiles are {vertex, first entry, end entry,
 // output row}, parts of one list each.
-template <int NB, bool TG, bool HUB>
-__global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const int4* tiles, int n_tiles,
+template <typename T, int NB, bool TG, bool HUB>
+__global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<T> a, const int4* tiles, int n_tiles,
                                                    const uint8_t* local, int CB, int nch, uint32_t table_bytes)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -92,6 +141,7 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
     constexpr int SHARE = 64 / GR;   // lanes that hold the same entry's lane_sums
     static_assert(NB <= 64 && NB % GR == 0, "a batch's entries sit one per lane");
     static_assert(NB / GR <= SHARE, "a lane keeps one of its groups' sums");
+    static_assert(!TG || sizeof(T) == 4, "lane_sums adds 32-bit lanes");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int B = a.B, Wy = a.Wy, k = a.k;
@@ -106,9 +156,9 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
         s_tab[x] = (uint8_t)(r < 0 ? 255 : 4 * r);
     }
     __syncthreads();
-    const uint32_t rowbytes = (uint32_t)a.lda * 4u;
+    const uint32_t rowbytes = (uint32_t)a.lda * (uint32_t)sizeof(T);
     const __amdgpu_buffer_rsrc_t table =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.aux), 0, (int)table_bytes, 0x00027000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.aux), 0, (int)table_bytes, 0x00027000);
     const int lane_coloring = lane / Wy;
     const uint8_t* tab = s_tab + (lane - lane_coloring * Wy);
     // a tile's chunks of colorings go to one XCD (workgroups are dealt to the 8
@@ -132,12 +182,12 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
             const bool mine = lane < nc * Wy;
             const int c = min(lane_coloring, nc - 1);
             const int shift = TG && !mine ? kStreamRowLanes * 4 : c * a.Wa * 4;  // (past the values: none)
-            const uint32_t place = lane < nc * a.Wa ? (uint32_t)(b0 * a.Wa + lane) * 4u : kStreamNoValue;
+            const uint32_t place = lane < nc * a.Wa ? (uint32_t)(b0 * a.Wa + lane) * (uint32_t)sizeof(T) : kStreamNoValue;
             const int nbat = (e1 - e0 + NB - 1) / NB;
             // lane j < NB holds entry j of a batch; one past the tile reads its
             // first entry with colours that add nothing
             int um = 0, lv = 0, lv_next = 0;
-            float wm = 1.0f;
+            T wm = T(1);
             bool last = false;
             uint32_t pd[kStreamColors / 4];
             uint32_t pt[3];
@@ -154,7 +204,7 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
                 const int ec = ok ? e : e0;
                 last = ok && (HUB ? e + 1 == e1 : lv_next != lv);
                 um = (int)((uint32_t)a.col[ec] * rowbytes);
-                wm = a.w && ok ? a.w[ec] : 1.0f;
+                wm = a.w && ok ? a.w[ec] : T(1);
                 const uint8_t* ep = a.ecol + (int64_t)ec * B + b0;
                 const uint8_t* vp = a.colors + (int64_t)(v0 + lv) * B + b0;
                 const uint32_t none = (uint32_t)(k * k);
@@ -174,20 +224,20 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
             locate(0);
             meta(0);
             if (nbat > 1) locate(1);
-            float acc = 0.0f;
+            T acc = T(0);
             int v = v0;
             // TG: the lane's values of the own rows of v and of the vertex after it
             auto own_row = [&](int u) {
-                return mine ? a.dy[(int64_t)min(u, v_last) * a.ldd + b0 * Wy + lane] : 0.0f;
+                return mine ? a.dy[(int64_t)min(u, v_last) * a.ldd + b0 * Wy + lane] : T(0);
             };
-            float own = 0.0f, own_next = 0.0f;
+            T own = T(0), own_next = T(0);
             if (TG) {
                 own = own_row(v0);
                 own_next = own_row(v0 + 1);
             }
             for (int t = 0; t < nbat; ++t) {
                 const int uc = um;
-                const float wc = wm;
+                const T wc = wm;
                 const uint64_t ends = __ballot(last);
                 unsigned char* to = s_pair + lane;
 #pragma unroll
@@ -199,17 +249,16 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
                 for (int r = 0; r < 3; ++r)
                     if (r < (nc & 3)) to[((nc & ~3) + r) * kStreamColorBytes] = (unsigned char)pt[r];
                 wave_sync();
-                float x[NB];
+                T x[NB];
 #pragma unroll
                 for (int j = 0; j < NB; ++j)
-                    x[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                        table, (int)place, __builtin_amdgcn_readlane(uc, j), 0));
+                    x[j] = table_value<T>(table, place, __builtin_amdgcn_readlane(uc, j));
                 if (t + 1 < nbat) {
                     meta(t + 1);  // the next batch's ids, behind this one's rows
                     if (t + 2 < nbat) locate(t + 2);
                 }
                 const unsigned char* from = s_pair + c * kStreamColorBytes;
-                float sums = 0.0f;
+                T sums = T(0);
                 // the lanes' values first, a group at a time, without a branch
                 // between them: their LDS reads and permutes overlap
 #pragma unroll
@@ -226,15 +275,15 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
                         at[j] = min((int)tab[__umul24((uint32_t)at[j], (uint32_t)Wy)] + shift, kStreamRowLanes * 4);
 #pragma unroll
                     for (int j = 0; j < GR; ++j)
-                        x[g + j] = __int_as_float(__builtin_amdgcn_ds_bpermute(at[j], __float_as_int(x[g + j])));
-                    float p[GR];  // TG: of the values without their weights
+                        x[g + j] = permuted(at[j], x[g + j]);
+                    T p[GR];  // TG: of the values without their weights
                     if (!TG && a.w)
 #pragma unroll
                         for (int j = 0; j < GR; ++j)
-                            x[g + j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wc), g + j)) * x[g + j];
+                            x[g + j] = lane_value(wc, g + j) * x[g + j];
                     auto scaled = [&](int j) {
                         if (!TG || !a.w) return x[g + j];
-                        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wc), g + j)) * x[g + j];
+                        return lane_value(wc, g + j) * x[g + j];
                     };
                     const uint32_t group_ends = (uint32_t)(ends >> g) & ((1u << GR) - 1u);
                     if (group_ends == 0) {
@@ -250,13 +299,13 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
                             if (TG) p[j] = own * x[g + j];
                             if ((group_ends >> j) & 1) {
                                 if (mine) {
-                                    float out = acc;
-                                    if (!TG && a.out_mode == OUT_EMA_SCALED) out = (float)((double)acc * (double)a.scale);
+                                    T out = acc;
+                                    if (!TG && a.out_mode == OUT_EMA_SCALED) out = (T)((double)acc * (double)a.scale);
                                     const int64_t row = HUB ? t4.w : v;
                                     a.out[row * a.ldo + b0 * Wy + lane] = out;
                                     if (!TG && a.ykeep) a.ykeep[(int64_t)v * a.ldy + b0 * Wy + lane] = acc;
                                 }
-                                acc = 0.0f;
+                                acc = T(0);
                                 ++v;
                                 if (TG && !HUB) {
                                     own = own_next;
@@ -266,7 +315,7 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
                         }
                     }
                     if constexpr (TG) {
-                        const float s = lane_sums(p, lane);
+                        const T s = lane_sums(p, lane);
                         if (lane % SHARE == g / GR) sums = s;
                     }
                 }
@@ -282,19 +331,20 @@ __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<float> a, const
     }
 }
 
-template <bool TG, bool HUB>
-hipError_t launch_stream_t(const SubArgs<float>& a, const int4* tiles, int n_tiles, const uint8_t* local,
+template <typename T, bool TG, bool HUB>
+hipError_t launch_stream_t(const SubArgs<T>& a, const int4* tiles, int n_tiles, const uint8_t* local,
                            uint32_t table_bytes, int num_cus, hipStream_t st)
 {
     const int most = stream_colorings(a.B, a.Wy, a.Wa);
     const int nch = (a.B + most - 1) / most;
     const int CB = (a.B + nch - 1) / nch;
+    constexpr int NB = kStreamBatch<T>;
     const size_t lds = stream_tab_bytes(a.k, a.Wy) + (size_t)(kBlock / 64) * kStreamColors * kStreamColorBytes;
     static thread_local std::map<size_t, int> per_cu_cache;
     auto it = per_cu_cache.find(lds);
     if (it == per_cu_cache.end()) {
         int per_cu = 0;
-        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stream<kStreamBatch, TG, HUB>, kBlock, lds);
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stream<T, NB, TG, HUB>, kBlock, lds);
         if (e != hipSuccess) return e;
         if (per_cu < 1) return hipErrorInvalidConfiguration;
         it = per_cu_cache.emplace(lds, per_cu).first;
@@ -302,7 +352,7 @@ hipError_t launch_stream_t(const SubArgs<float>& a, const int4* tiles, int n_til
     const int64_t need = ((int64_t)n_tiles * (TG ? 1 : nch) + kBlock / 64 - 1) / (kBlock / 64);
     const int64_t most_blocks = std::min<int64_t>(need, (int64_t)it->second * num_cus);
     const int grid = (int)((most_blocks + kXcds - 1) / kXcds) * kXcds;
-    hipLaunchKernelGGL((k_stream<kStreamBatch, TG, HUB>), dim3(grid), dim3(kBlock), lds, st, a, tiles, n_tiles, local, CB, nch,
+    hipLaunchKernelGGL((k_stream<T, NB, TG, HUB>), dim3(grid), dim3(kBlock), lds, st, a, tiles, n_tiles, local, CB, nch,
                        table_bytes);
     return hipGetLastError();
 }
@@ -314,25 +364,34 @@ int stream_colorings(int B, int Wy, int Wa)
     return std::min({B, 64 / Wy, kStreamRowLanes / Wa, kStreamColors});
 }
 
-bool stream_fits(int64_t n_rows, int lda, int Wy, int Wa)
+bool stream_fits(int64_t n_rows, int64_t row_bytes, int Wy, int Wa)
 {
-    return Wy >= 1 && Wy <= 64 && Wa >= 1 && Wa <= kStreamRowLanes && n_rows * lda * 4 <= (int64_t)kStreamNoValue;
+    return Wy >= 1 && Wy <= 64 && Wa >= 1 && Wa <= kStreamRowLanes && n_rows * row_bytes <= (int64_t)kStreamNoValue;
 }
 
-hipError_t launch_stream(StreamMode mode, const SubArgs<float>& a, const int4* tiles, int n_tiles,
-                         const uint8_t* local, int64_t n_rows, int num_cus, hipStream_t st)
+template <typename T>
+hipError_t launch_stream(StreamMode mode, const SubArgs<T>& a, const int4* tiles, int n_tiles, const uint8_t* local,
+                         int64_t n_rows, int num_cus, hipStream_t st)
 {
     if (n_tiles <= 0) return hipSuccess;
-    if (a.k > kMaxK || !a.gidx || !stream_fits(n_rows, a.lda, a.Wy, a.Wa)) return hipErrorInvalidValue;
-    const uint32_t bytes = (uint32_t)(n_rows * a.lda * 4);
+    const int64_t row_bytes = (int64_t)a.lda * (int64_t)sizeof(T);
+    if (a.k > kMaxK || !a.gidx || !stream_fits(n_rows, row_bytes, a.Wy, a.Wa)) return hipErrorInvalidValue;
+    const uint32_t bytes = (uint32_t)(n_rows * row_bytes);
     if (mode == STREAM_FORWARD) {
         if (a.out_mode != OUT_EMA && a.out_mode != OUT_EMA_SCALED) return hipErrorInvalidValue;
-        return launch_stream_t<false, false>(a, tiles, n_tiles, local, bytes, num_cus, st);
+        return launch_stream_t<T, false, false>(a, tiles, n_tiles, local, bytes, num_cus, st);
     }
-    if (!a.dy || !a.grad || (a.out_mode != OUT_Y && a.out_mode != OUT_PARTIAL)) return hipErrorInvalidValue;
-    return mode == STREAM_TG ? launch_stream_t<true, false>(a, tiles, n_tiles, local, bytes, num_cus, st)
-                             : launch_stream_t<true, true>(a, tiles, n_tiles, local, bytes, num_cus, st);
+    if constexpr (sizeof(T) == 4)
+        if (a.dy && a.grad && (a.out_mode == OUT_Y || a.out_mode == OUT_PARTIAL))
+            return mode == STREAM_TG ? launch_stream_t<T, true, false>(a, tiles, n_tiles, local, bytes, num_cus, st)
+                                     : launch_stream_t<T, true, true>(a, tiles, n_tiles, local, bytes, num_cus, st);
+    return hipErrorInvalidValue;
 }
+
+template hipError_t launch_stream<float>(StreamMode, const SubArgs<float>&, const int4*, int, const uint8_t*, int64_t, int,
+                                         hipStream_t);
+template hipError_t launch_stream<double>(StreamMode, const SubArgs<double>&, const int4*, int, const uint8_t*, int64_t,
+                                          int, hipStream_t);
 
 __global__ void k_local_ids(uint8_t* local, const int4* tiles, int n_tiles, const int32_t* rowptr)
 {
