@@ -1998,6 +1998,37 @@ GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
     return g;
 }
 
+// The dY of steps with a leaf aux child whose entries' gradients wait for a
+// common launch, in step order.
+template <typename T>
+struct LeafGrads {
+    const T* dY[kEdgeGradSteps];
+    int n = 0;
+    int32_t Wy = 0;      // of every such step: k - 1, the single other colours
+    double bytes = 0.0;  // their byte models
+};
+
+template <typename T>
+int enqueue_leaf_grads(pg_ctx* c, int B, const PassBufs<T>& pb, LeafGrads<T>& leaf)
+{
+    if (leaf.n == 0) return PG_OK;
+    EdgeGradArgs<T> eg{};
+    eg.nnz = c->nnz;
+    eg.B = B;
+    eg.erow = c->d_erow.as<int32_t>();
+    eg.colors = pb.colors;
+    eg.ecol = pb.ecol;
+    std::copy(leaf.dY, leaf.dY + leaf.n, eg.dY);
+    eg.n_steps = leaf.n;
+    eg.Wy = leaf.Wy;
+    eg.grad = c->d_grad.as<double>();
+    record(c, sizeof(T) == 4 ? "k_edge_grad<float>" : "k_edge_grad<double>", leaf.bytes, true);
+    HIP_TRY(c, launch_edge_grad<T>(eg, c->stream));
+    record(c, "", 0, false);
+    leaf = LeafGrads<T>{};
+    return PG_OK;
+}
+
 // The backward step of one subtemplate d: from G_s (nullptr at the root,
 // whose cotangents are cot), the main and aux children's tables Tm / Ta,
 // write G_main into Gm and G_aux into Ga (nullptr for leaf children), and add
@@ -2010,10 +2041,12 @@ GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
 // forms dY and G_main together from it, and the transposed gather also takes
 // the entries' gradients (RUNS_TG): no gradient gather, no second read of
 // the aux rows.
+//
+// A step with a leaf aux child leaves its entries' gradients to `leaf`.
 template <typename T>
 int enqueue_sub_backward(pg_ctx* c, const pg_plan* p, const DevSub& d, int B, const PassBufs<T>& pb, T* Ybuf,
                          T* dYbuf, const double* cot, const T* Tm, const T* Ta, const T* G, T* Gm, T* Ga,
-                         const T* Yk = nullptr)
+                         LeafGrads<T>& leaf, const T* Yk = nullptr)
 {
     const SubTag tag(c, d.s);
     const hipStream_t st = c->stream;
@@ -2141,28 +2174,11 @@ int enqueue_sub_backward(pg_ctx* c, const pg_plan* p, const DevSub& d, int B, co
             HIP_TRY(c, launch_bwd_node<T>(na, c->num_cus, st));
             record(c, "", 0, false);
         }
-        EdgeGradArgs<T> eg{};
-        eg.nnz = c->nnz;
-        eg.B = B;
-        eg.k = p->k;
-        eg.K = p->K;
-        eg.erow = c->d_erow.as<int32_t>();
-        eg.col = c->d_col.as<int32_t>();
-        eg.colors = pb.colors;
-        eg.ecol = pb.ecol;
-        eg.dY = dYin;
-        eg.Wy = d.Wy;
-        eg.Ta = nullptr;
-        eg.Wa = d.Wa;
-        eg.ymask = d.ymask.as<uint16_t>();
-        eg.rank_tab = p->rank_tab.as<int16_t>();
-        eg.grad = c->d_grad.as<double>();
         // entry rows and columns, the neighbour colors (a byte per entry and
         // coloring), the vertex colors, dY, and the gradient
-        record(c, std::string("k_edge_grad<") + (fp32 ? "float>" : "double>"),
-               8.0 * Z + Z * B + (double)c->n_act * B + col * Ca + 16.0 * Z, true);
-        HIP_TRY(c, launch_edge_grad<T>(eg, st));
-        record(c, "", 0, false);
+        leaf.dY[leaf.n++] = dYin;
+        leaf.Wy = d.Wy;
+        leaf.bytes += 8.0 * Z + Z * B + (double)c->n_act * B + col * Ca + 16.0 * Z;
     }
     return PG_OK;
 }
@@ -2175,17 +2191,32 @@ int enqueue_backward_kept(pg_ctx* c, const pg_plan* p, int B, const GradPlan& gp
     const PassBufs<T> pb = pass_bufs<T>(c, gp.fwd);
     auto tab = [&](int s) { return (T*)(base + gp.fwd.off_tab[s]); };
     auto gad = [&](int s) { return (T*)(base + gp.off_G[s]); };
+    T* const dYbuf = (T*)(base + gp.off_dY);
+    LeafGrads<T> leaf;
+    bool waits_in_dYbuf = false;
     for (auto it = p->subs.rbegin(); it != p->subs.rend(); ++it) {
         const DevSub& d = **it;
         const size_t yk = (size_t)d.s < gp.fwd.off_ykeep.size() ? gp.fwd.off_ykeep[d.s] : 0;
-        int rc = enqueue_sub_backward<T>(c, p, d, B, pb, (T*)(base + gp.off_Y), (T*)(base + gp.off_dY),
-                                         (const double*)(base + gp.off_cot), d.mm > 1 ? tab(d.mi) : nullptr,
-                                         d.aa > 1 ? tab(d.ai) : nullptr, d.root ? nullptr : gad(d.s),
-                                         d.mm > 1 ? gad(d.mi) : nullptr, d.aa > 1 ? gad(d.ai) : nullptr,
-                                         yk ? (const T*)(base + yk) : nullptr);
+        // A leaf aux child's dY waits for the common launch in the step's own
+        // forward table, which only the steps above it, done by now, read; the
+        // root, which has none, uses the common buffer.
+        const bool own = d.aa == 1 && !d.root && d.Wo >= d.Wy;
+        T* const dY = own ? tab(d.s) : dYbuf;
+        int rc = PG_OK;
+        if (leaf.n == kEdgeGradSteps || (!own && waits_in_dYbuf)) {
+            rc = enqueue_leaf_grads<T>(c, B, pb, leaf);
+            if (rc) return rc;
+            waits_in_dYbuf = false;
+        }
+        if (d.aa == 1 && !own) waits_in_dYbuf = true;
+        rc = enqueue_sub_backward<T>(c, p, d, B, pb, (T*)(base + gp.off_Y), dY,
+                                     (const double*)(base + gp.off_cot), d.mm > 1 ? tab(d.mi) : nullptr,
+                                     d.aa > 1 ? tab(d.ai) : nullptr, d.root ? nullptr : gad(d.s),
+                                     d.mm > 1 ? gad(d.mi) : nullptr, d.aa > 1 ? gad(d.ai) : nullptr,
+                                     leaf, yk ? (const T*)(base + yk) : nullptr);
         if (rc) return rc;
     }
-    return PG_OK;
+    return enqueue_leaf_grads<T>(c, B, pb, leaf);
 }
 
 // First-fit allocator of byte ranges in [0, cap) of the pool (host-side
@@ -2266,7 +2297,11 @@ struct Recompute {
             return PG_ERR_NOMEM;
         if (d.aa > 1 && (ga = pool.alloc(table_bytes(c, *sub[d.ai], B, sizeof(T)))) == PoolAlloc::kNone)
             return PG_ERR_NOMEM;
-        if (!dry) rc = enqueue_sub_backward<T>(c, p, d, B, pb, Ybuf, dYbuf, cot, at(tm), at(ta), at(g), at(gm), at(ga));
+        if (!dry) {
+            LeafGrads<T> leaf;
+            rc = enqueue_sub_backward<T>(c, p, d, B, pb, Ybuf, dYbuf, cot, at(tm), at(ta), at(g), at(gm), at(ga), leaf);
+            if (rc == PG_OK) rc = enqueue_leaf_grads<T>(c, B, pb, leaf);
+        }
         if (rc) return rc;
         pool.release(tm);
         pool.release(ta);

@@ -300,22 +300,19 @@ constexpr size_t kNodeRows16Lds = 80 * 1024 - 64;
 size_t node_rows16_lds_bytes(const NodeArgs<float>& a);
 hipError_t launch_bwd_node_rows16(const NodeArgs<float>& a, int num_cus, hipStream_t st);
 
-// Per entry e = (row v, column u): grad[e] += sum_b sum_i dY[v][b][i] * T_a-term(u)
-// (aux table) or dY[v][b][i(col u)] (aux leaf).  One thread per entry.
+// Per entry e = (row v, column u) and step s with a leaf aux child:
+// grad[e] += sum_b dY[s][v][b][i(col u)].  One thread per entry.
+constexpr int kEdgeGradSteps = 4;
 template <typename T>
 struct EdgeGradArgs {
     int64_t nnz;
-    int32_t B, k, K;
+    int32_t B;
     const int32_t* erow;     // [nnz] row (internal vertex) of each entry
-    const int32_t* col;
     const uint8_t* colors;   // [n_act][B]
     const uint8_t* ecol;     // [nnz][B]
-    const T* dY;             // [n_act][B*Wy]
+    const T* dY[kEdgeGradSteps];  // [n_act][B*Wy] of each step
+    int32_t n_steps;
     int32_t Wy;
-    const T* Ta;             // [n_act][B*Wa] (aux not a leaf), nullptr for a leaf aux
-    int32_t Wa;
-    const uint16_t* ymask;   // [Wy]
-    const int16_t* rank_tab;
     double* grad;            // [nnz] internal order, accumulated
 };
 template <typename T>
