@@ -414,8 +414,11 @@ def headline(args, sync):
                     "one coloring (stream seed 4242, coloring 0) of the headline graph and template: the whole "
                     "12-vertex-tree DP of CountMat::colorCounting (forward only; the reference has no adjoint)")
             cb = result["cpu_baseline"]
-            log(f"cpu: {cb['value']:.4f} colorings/s on {cb['cores']} threads ({cb['cpu_model']}), parity max rel "
-                f"err {cb['parity_max_rel_err']:.2e}")
+            if cb["value"] is None:
+                log(f"cpu: {cb['sample']}")
+            else:
+                log(f"cpu: {cb['value']:.4f} colorings/s on {cb['cores']} threads ({cb['cpu_model']}), parity max rel "
+                    f"err {cb['parity_max_rel_err']:.2e}")
         except (subprocess.SubprocessError, OSError) as e:
             result["cpu_baseline"] = {"value": None, "unit": "colorings/s", "cores": physical_cores(),
                                       "kind": "reference", "sample": f"failed: {e}"}
@@ -544,8 +547,11 @@ def plain_s20(args, sync):
                     gp, 7, TREE7, seed, args.cpu_colorings, lambda c: ctx.count(plan, c, seed=seed).tolist(),
                     f"{args.cpu_colorings} colorings (stream seed {seed}) of this workload")
             cb = out["cpu_baseline"]
-            log(f"plain s20 cpu: {cb['value']:.3f} colorings/s on {cb['cores']} threads, parity "
-                f"{cb['parity_max_rel_err']:.2e}")
+            if cb["value"] is None:
+                log(f"plain s20 cpu: {cb['sample']}")
+            else:
+                log(f"plain s20 cpu: {cb['value']:.3f} colorings/s on {cb['cores']} threads, parity "
+                    f"{cb['parity_max_rel_err']:.2e}")
         except (subprocess.SubprocessError, OSError) as e:
             out["cpu_baseline"] = {"value": None, "sample": f"failed: {e}"}
     return out
@@ -725,8 +731,10 @@ def record_name(symbol):
         s = s.replace(junk, "")
     m = re.match(r"(k_\w+)<(.*)>$", s)
     if not m:
-        return "k_combine_rows<float>" if s == "k_combine_rows" else s
+        return {"k_combine_rows": "k_combine_rows<float>", "k_edge_colors_word": "k_edge_colors"}.get(s, s)
     name, a = m.group(1), m.group(2).split(",")
+    if name == "k_edge_colors":
+        return name
     if name == "k_sub" and len(a) == 5:
         return "k_sub<" + ",".join(a[:4] + ([] if a[4] == "4" else ["1"])) + ">"
     if name in ("k_hub_seq", "k_root_seq"):
