@@ -183,7 +183,7 @@ struct pg_ctx {
     // adjoint support, built on first use: row of each entry, the entry of
     // the transposed pair, and weights in transposed order
     bool has_transpose = false, symmetric = false;
-    DevBuf d_erow, d_tr, d_wT32, d_wT64, d_grad, d_grad_out;
+    DevBuf d_erow, d_tr, d_ent_tr, d_wT32, d_wT64, d_grad, d_grad_out;
     DevBuf d_rowptr, d_col, d_ent, d_perm, d_w32, d_w64, d_wsrc;
     bool w64_filled = false;  // d_w64 holds the current weights (widened from d_w32 for the first FP64 pass)
     // degree buckets and hub work items for the current options
@@ -824,7 +824,7 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
                      int used_per_mille = 0)
 {
     {
-        if (a.tr) {  // the fused transposed gather and gradient (fused_grad_step)
+        if (a.own) {  // the fused transposed gather and gradient (fused_grad_step)
             if (runs_values_per_lane(a.Wa) == 0) return set_err(c, PG_ERR_STATE, "fused gradient gather too wide");
             return launch_gathering_runs<T>(c, RUNS_TG, main_mode, a, part, y_cols, bytes);
         }
@@ -1889,6 +1889,11 @@ int build_transpose(pg_ctx* c)
     HIP_TRY(c, c->d_tr.alloc(tr.size() * 4));
     HIP_TRY(c, hipMemcpy(c->d_erow.p, erow.data(), erow.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(c, hipMemcpy(c->d_tr.p, tr.data(), tr.size() * 4, hipMemcpyHostToDevice));
+    if (c->symmetric) {
+        HIP_TRY(c, c->d_ent_tr.alloc(tr.size() * 4));
+        HIP_TRY(c, launch_gather_ids(c->d_ent_tr.as<int32_t>(), c->d_ent.as<int32_t>(), c->d_tr.as<int32_t>(), nnz,
+                                     c->stream));
+    }
     c->has_transpose = true;
     return PG_OK;
 }
@@ -2120,9 +2125,8 @@ int enqueue_sub_backward(pg_ctx* c, const pg_plan* p, const DevSub& d, int B, co
         const StepBytes bytes{csc_bytes(c), col * Ca + 20.0 * Z, col * 2.0 * Ca};
         t.own = Ta;
         t.ldown = B * d.Wa;
-        t.tr = c->d_tr.as<int32_t>();
         t.ttab = d.ttab.as<int16_t>();
-        t.grad = c->d_grad.as<double>();
+        t.grad = c->d_grad.as<double>() + c->nnz;  // of the transposed entries
         return launch_gathering<T>(c, AUX_GATHER_T, MAIN_LEAF, t, pb.part, B * d.Wa, bytes,
                                    runs_used_per_mille(p, d, AUX_GATHER_T));
     }
@@ -2449,9 +2453,9 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         HIP_TRY(c, launch_gather_weights<T>(wT.as<T>(), c->d_w32.as<float>(), c->d_tr.as<int32_t>(), c->nnz, c->stream));
     }
     // the entries' gradients and, where a transposed gather takes them in list
-    // order (AUX_GATHER_TG), those of their transposes
+    // order (AUX_GATHER_TG, RUNS_TG), those of their transposes
     bool by_transpose = false;
-    for (auto& d : p->subs) by_transpose |= lane_grad_step(c, p, *d);
+    for (auto& d : p->subs) by_transpose |= lane_grad_step(c, p, *d) || fused_grad_step(c, p, *d);
     const int64_t n_acc = c->nnz * (by_transpose ? 2 : 1);
     HIP_TRY(c, c->d_grad.alloc(std::max<int64_t>(n_acc, 1) * 8));
     HIP_TRY(c, launch_zero_f64(c->d_grad.as<double>(), n_acc, c->stream));
@@ -2553,16 +2557,17 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         if (grad_on_device) {
             if (sizeof(T) == 4)
                 HIP_TRY(c, launch_scatter_grad<float>((float*)grad, c->d_grad.as<double>(), g_tr, c->d_tr.as<int32_t>(),
-                                                      c->d_ent.as<int32_t>(), c->nnz, factor, c->stream));
+                                                      c->d_ent.as<int32_t>(), c->d_ent_tr.as<int32_t>(), c->nnz, factor,
+                                                      c->stream));
             else
                 HIP_TRY(c, launch_scatter_grad<double>((double*)grad, c->d_grad.as<double>(), g_tr,
-                                                       c->d_tr.as<int32_t>(), c->d_ent.as<int32_t>(), c->nnz, factor,
-                                                       c->stream));
+                                                       c->d_tr.as<int32_t>(), c->d_ent.as<int32_t>(),
+                                                       c->d_ent_tr.as<int32_t>(), c->nnz, factor, c->stream));
         } else {
             HIP_TRY(c, c->d_grad_out.alloc(std::max<int64_t>(c->nnz, 1) * 8));
             HIP_TRY(c, launch_scatter_grad<double>(c->d_grad_out.as<double>(), c->d_grad.as<double>(), g_tr,
-                                                   c->d_tr.as<int32_t>(), c->d_ent.as<int32_t>(), c->nnz, factor,
-                                                   c->stream));
+                                                   c->d_tr.as<int32_t>(), c->d_ent.as<int32_t>(),
+                                                   c->d_ent_tr.as<int32_t>(), c->nnz, factor, c->stream));
             HIP_TRY(c, hipMemcpyAsync(grad, c->d_grad_out.p, c->nnz * 8, hipMemcpyDeviceToHost, c->stream));
         }
     }

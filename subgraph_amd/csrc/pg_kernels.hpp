@@ -118,11 +118,10 @@ struct SubArgs {
     int32_t ldd;             // dy row stride (B * Wy)
     double* grad;            // [nnz] internal entry order
     // RUNS_TG (the transposed gather fused with the gradient): the vertex's
-    // own row of the aux child's table, and the transposed entry of each
-    // entry, whose gradient the neighbour's dY row dotted with it gives
+    // own row of the aux child's table; the neighbour's dY row dotted with it
+    // gives the gradient of the transposed entry
     const T* own;            // [n_act][ldown]
     int32_t ldown;           // B * (aux child's row width)
-    const int32_t* tr;       // [nnz] entry (u, v) of entry (v, u)
     // ttab[((cv * k + c) * 64 + lane) * RV + t]: the entry of the vertex's
     // row (colour cv) that position lane + 64 t of a neighbour's dY row
     // (colour c) adds to, or -1; RV = runs_values_per_lane(dY width)
@@ -182,7 +181,7 @@ hipError_t launch_sub(int team, int aux, int main_mode, int rc, const SubArgs<T>
 // neighbour through xidx (every (vertex colour, neighbour colour) row of it),
 // a team per (vertex, colouring) with the whole neighbour list.
 // RUNS_TG is RUNS_T plus, for every entry (v, u) of the vertex's list, the
-// gradient of its transpose: grad[tr[e]] += dY[u] . (own row of v mapped to
+// gradient of its transpose: grad[e] += dY[u] . (own row of v mapped to
 // u's Y positions), a team per item with every coloring in order.
 enum RunsMode : int { RUNS_FWD = 0, RUNS_T = 1, RUNS_G = 2, RUNS_SEQ = 3, RUNS_TG = 4 };
 // values per lane for a gathered row of wg values (0: too wide)
@@ -318,10 +317,13 @@ struct EdgeGradArgs {
 template <typename T>
 hipError_t launch_edge_grad(const EdgeGradArgs<T>& a, hipStream_t st);
 
-// out[ent[i]] = (TO) (factor * (grad[i] + grad_tr[tr[i]])); grad_tr nullptr: grad alone
+// out[ent[i]] = (TO) (factor * grad[i]); with grad_tr, the gradients of the
+// entries' transposes, out[ent_tr[i]] = (TO) (factor * (grad[tr[i]] + grad_tr[i]))
 template <typename TO>
 hipError_t launch_scatter_grad(TO* out, const double* grad, const double* grad_tr, const int32_t* tr, const int32_t* ent,
-                               int64_t nnz, double factor, hipStream_t st);
+                               const int32_t* ent_tr, int64_t nnz, double factor, hipStream_t st);
+// dst[i] = ids[at[i]]
+hipError_t launch_gather_ids(int32_t* dst, const int32_t* ids, const int32_t* at, int64_t n, hipStream_t st);
 hipError_t launch_zero_f64(double* p, int64_t n, hipStream_t st);
 
 // ---- the reference's unpruned mode (isPruned = 0, CountMat.cpp:851-977) ----

@@ -530,7 +530,9 @@ __global__ __launch_bounds__(kBlock) void k_runs_g(const SubArgs<T> a)
 // col(v)).  That entry is also where the vertex's own aux-child row enters
 // the neighbour's Y value A_t, so for each neighbour u the team dots u's dY
 // row with its own row mapped the same way: d Y[u] / d w_(u,v) . dY[u], the
-// gradient of the transposed entry (u, v), added to grad[tr[e]] in FP64.
+// gradient of the transposed entry (u, v), added to grad[e] of the transposed
+// entries' array in FP64 (in list order: entry tr[e] of the other array is a
+// line of memory read and written at random per entry and coloring).
 // With the forward's Y kept, this replaces the gradient gather (RUNS_G) and
 // its second read of the aux rows.
 //
@@ -604,10 +606,8 @@ void k_runs_tg(const SubArgs<T> a)
                     const int ee = w0 + lane;
                     const bool ok = ee < e1;
                     const uint32_t cc = ok ? (uint32_t)a.ecol[(int64_t)ee * B + b] : kNone;
-                    // the entry's neighbour, transposed entry and weight load
-                    // beside its colour
+                    // the entry's neighbour and weight load beside its colour
                     const int uid = ok ? a.col[ee] : 0;
-                    const int tre = ok ? a.tr[ee] : 0;
                     const T wv = ok && a.w ? a.w[ee] : T(1);
                     const bool use = ok && cc != cv;
                     int pos = 0, n = 0;
@@ -618,7 +618,7 @@ void k_runs_tg(const SubArgs<T> a)
                         n += __popcll(m);
                     }
                     if (use) {
-                        sQ[pos] = make_int4(uid, tre, (int)cc, 0);
+                        sQ[pos] = make_int4(uid, ee, (int)cc, 0);
                         sW[pos] = wv;
                     }
                     wave_sync();
@@ -1028,8 +1028,8 @@ hipError_t launch_runs(int mode, int main_mode, const SubArgs<T>& a, int num_cus
         return launch_runs_rv<T, RUNS_T, MAIN_LEAF>(rv, a, num_cus, blocks_per_cu, st);
     }
     if (mode == RUNS_TG) {
-        if (main_mode != MAIN_LEAF || (a.out_mode != OUT_Y && a.out_mode != OUT_PARTIAL) || !a.own || !a.tr ||
-            !a.grad || !a.ttab)
+        if (main_mode != MAIN_LEAF || (a.out_mode != OUT_Y && a.out_mode != OUT_PARTIAL) || !a.own || !a.grad ||
+            !a.ttab)
             return hipErrorInvalidValue;
         switch (rv) {
         case 1: return launch_runs_tg_t<T, 1>(a, num_cus, blocks_per_cu, st);
