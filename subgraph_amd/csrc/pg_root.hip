@@ -40,7 +40,9 @@ __global__ __launch_bounds__(kBlock) void k_root_seq(const SubArgs<T> a, const i
         T carry = T(0);  // a lone vertex may have more entries than a tile holds
         for (int b0 = 0; b0 < B; b0 += C) {
             const int nc = min(C, B - b0);
-            for (int w0 = 0; w0 < ne; w0 += kRootTileEntries) {
+            // (once for a tile without entries: its vertices' sums are zero)
+            int w0 = 0;
+            do {
                 const int nw = min(kRootTileEntries, ne - w0);
                 __syncthreads();
                 for (int e = tid; e < nw; e += kBlock) {
@@ -92,7 +94,8 @@ __global__ __launch_bounds__(kBlock) void k_root_seq(const SubArgs<T> a, const i
                     // f32 product y * 1, widened (DataTableColMajor.cpp:396)
                     if (w0 + nw >= ne) a.root_vals[(int64_t)(b0 + c) * a.n_root + v0 + j] = (double)acc;
                 }
-            }
+                w0 += kRootTileEntries;
+            } while (w0 < ne);
         }
     }
 }
