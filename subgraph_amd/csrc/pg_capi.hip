@@ -178,6 +178,7 @@ struct pg_ctx {
     // graph
     bool has_graph = false, weighted = false;
     int32_t n = 0, n_act = 0, max_deg = 0;
+    int32_t n_full = 0;  // leading vertices with a neighbour list; the others occur as columns only
     int64_t nnz = 0;
     std::vector<int32_t> h_rowptr, h_col, h_perm;
     // adjoint support, built on first use: row of each entry, the entry of
@@ -318,13 +319,14 @@ int build_buckets(pg_ctx* c)
         HIP_TRY(c, c->d_hub_iota.alloc(iota.size() * sizeof(int32_t)));
         HIP_TRY(c, hipMemcpy(c->d_hub_iota.p, iota.data(), iota.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     }
-    // tiles of the vertices below the hubs: consecutive ones within both limits
-    auto make_tiles = [&](int max_entries, int max_vertices, DevBuf& buf, int& n, std::vector<int32_t>* first) -> int {
+    // tiles of the vertices [nh, end) below the hubs: consecutive ones within both limits
+    auto make_tiles = [&](int32_t end, int max_entries, int max_vertices, DevBuf& buf, int& n,
+                          std::vector<int32_t>* first) -> int {
         std::vector<int4> tiles;
-        for (int32_t v = nh; v < c->n_act;) {
+        for (int32_t v = nh; v < end;) {
             const int32_t e = c->h_rowptr[v];
             int32_t w = v + 1;
-            while (w < c->n_act && w - v < max_vertices && c->h_rowptr[w + 1] - e <= max_entries) ++w;
+            while (w < end && w - v < max_vertices && c->h_rowptr[w + 1] - e <= max_entries) ++w;
             tiles.push_back(make_int4(v, w - v, e, c->h_rowptr[w] - e));
             if (first) first->push_back(v);
             v = w;
@@ -334,10 +336,12 @@ int build_buckets(pg_ctx* c)
         if (!tiles.empty()) HIP_TRY(c, hipMemcpy(buf.p, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
         return PG_OK;
     };
-    int rc = make_tiles(kRootTileEntries, kRootTileVertices, c->d_root_tiles, c->n_root_tiles, nullptr);
+    int rc = make_tiles(c->n_act, kRootTileEntries, kRootTileVertices, c->d_root_tiles, c->n_root_tiles, nullptr);
     if (rc) return rc;
     c->h_stream_first.clear();
-    rc = make_tiles(kStreamTileEntries, kStreamTileVertices, c->d_stream_tiles, c->n_stream_tiles, &c->h_stream_first);
+    // (k_stream stores a sum where an entry ends a list: no empty ones)
+    rc = make_tiles(c->n_full, kStreamTileEntries, kStreamTileVertices, c->d_stream_tiles, c->n_stream_tiles,
+                    &c->h_stream_first);
     if (rc) return rc;
     HIP_TRY(c, c->d_local.alloc(std::max<int64_t>(c->nnz, 1)));
     HIP_TRY(c, launch_local_ids(c->d_local.as<uint8_t>(), c->d_stream_tiles.as<int4>(), c->n_stream_tiles,
@@ -928,7 +932,7 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
 }
 
 // the first streaming tile that starts at vertex v or later, and the last
-// vertex in [v0, v] that starts a tile (v itself where the tiles end)
+// vertex in [v0, v] that starts a tile (v itself past the tiles)
 int tile_of(const pg_ctx* c, int32_t v)
 {
     const auto& f = c->h_stream_first;
@@ -938,7 +942,7 @@ int tile_of(const pg_ctx* c, int32_t v)
 int32_t tile_floor(const pg_ctx* c, int32_t v0, int32_t v)
 {
     const auto& f = c->h_stream_first;
-    if (v >= c->n_act) return v;
+    if (v >= c->n_full) return v;
     const auto it = std::upper_bound(f.begin(), f.end(), v);
     return it == f.begin() ? v0 : std::max(v0, *(it - 1));
 }
@@ -1024,6 +1028,9 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
             record(c, sizeof(T) == 4 ? "k_stream<float>" : "k_stream<double>", sh, true);
             HIP_TRY(c, launch_stream<T>(STREAM_FORWARD, r, c->d_stream_tiles.as<int4>() + t0, t1 - t0,
                                         c->d_local.as<uint8_t>(), c->n_act, cus, rs));
+            // the sums of empty lists (a step whose Y is kept has none: its pattern is symmetric)
+            const int32_t z = std::max(v0, c->n_full);
+            if (z < v1) HIP_TRY(c, launch_zero<T>(r.out + (int64_t)z * r.ldo, (int64_t)(v1 - z) * r.ldo, rs));
         } else if (root_tiles) {
             record(c, sizeof(T) == 4 ? "k_root_seq<float>" : "k_root_seq<double>", sh, true);
             HIP_TRY(c, launch_root_seq<T>(r, c->d_root_tiles.as<int4>(), c->n_root_tiles, cus, rs));
@@ -2458,7 +2465,7 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
     for (auto& d : p->subs) by_transpose |= lane_grad_step(c, p, *d) || fused_grad_step(c, p, *d);
     const int64_t n_acc = c->nnz * (by_transpose ? 2 : 1);
     HIP_TRY(c, c->d_grad.alloc(std::max<int64_t>(n_acc, 1) * 8));
-    HIP_TRY(c, launch_zero_f64(c->d_grad.as<double>(), n_acc, c->stream));
+    HIP_TRY(c, launch_zero<double>(c->d_grad.as<double>(), n_acc, c->stream));
     const double* g_tr = by_transpose ? c->d_grad.as<double>() + c->nnz : nullptr;
     const uint8_t* d_in = nullptr;
     if (colors) {
@@ -2939,7 +2946,8 @@ extern "C" int pg_get_option(const pg_ctx* c, const char* key, int64_t* v)
 // Internal order: vertices that appear in any entry, by descending row
 // degree (ties by caller id), so hubs form a prefix, degree buckets are
 // ranges, and isolated vertices -- whose tables are all zero above the
-// leaves -- are dropped.  Row v lists the entries (row v, column u) in
+// leaves -- are dropped.  Vertices that occur as columns only, whose lists are
+// empty, come last.  Row v lists the entries (row v, column u) in
 // ascending u, the order in which the reference accumulates row v
 // (CSCGraph.hpp:199-213, 254-307).
 extern "C" int pg_graph_upload(pg_ctx* c, int32_t n, int64_t nnz, const int32_t* colptr, const int32_t* rowidx,
@@ -3010,8 +3018,8 @@ extern "C" int pg_graph_upload(pg_ctx* c, int32_t n, int64_t nnz, const int32_t*
                 }
             }
         }
-        // degree >= bound: hubs above 128, 256, 512, 1024; team buckets from 4 .. 512
-        static const int64_t bounds[] = {1025, 513, 512, 257, 256, 129, 128, 64, 32, 16, 8, 4};
+        // degree >= bound: hubs above 128, 256, 512, 1024; team buckets from 4 .. 512; a list at all
+        static const int64_t bounds[] = {1025, 513, 512, 257, 256, 129, 128, 64, 32, 16, 8, 4, 1};
         auto cls = [&](int32_t v) {
             int k = 0;
             for (int64_t b : bounds) {
@@ -3045,6 +3053,8 @@ extern "C" int pg_graph_upload(pg_ctx* c, int32_t n, int64_t nnz, const int32_t*
     c->n_act = na;
     c->max_deg = 0;
     for (int32_t v : perm) c->max_deg = std::max(c->max_deg, rdeg[v]);
+    c->n_full = 0;
+    while (c->n_full < na && hrow[c->n_full + 1] > hrow[c->n_full]) ++c->n_full;
     c->h_rowptr = hrow;
     c->h_col = hcol;
     c->h_perm = perm;

@@ -480,7 +480,8 @@ __global__ __launch_bounds__(kBlock) void k_sub(const SubArgs<T> a)
                     // software pipeline: the ids, colors and weights of the
                     // next 4 neighbours load while the current rows are read.
                     // Loads are unconditional: an entry past the end reads the
-                    // item's last entry (which exists) and is flagged.  With
+                    // item's last entry (of an empty list, which comes after all
+                    // others, the graph's last) and is flagged.  With
                     // gidx the flag only moves the table base to the all -1
                     // rows, so no loaded value feeds a select (which would let
                     // the compiler sink the loads under branches).
@@ -1529,16 +1530,21 @@ hipError_t launch_gather_ids(int32_t* dst, const int32_t* ids, const int32_t* at
     return hipGetLastError();
 }
 
-__global__ void k_zero_f64(double* p, int64_t n)
+template <typename T>
+__global__ void k_zero(T* p, int64_t n)
 {
-    FLAT_LOOP(i, n) p[i] = 0.0;
+    FLAT_LOOP(i, n) p[i] = T(0);
 }
 
-hipError_t launch_zero_f64(double* p, int64_t n, hipStream_t st)
+template <typename T>
+hipError_t launch_zero(T* p, int64_t n, hipStream_t st)
 {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_zero_f64, flat_grid(n), dim3(256), 0, st, p, n);
+    hipLaunchKernelGGL(k_zero<T>, flat_grid(n), dim3(256), 0, st, p, n);
     return hipGetLastError();
 }
+
+template hipError_t launch_zero<float>(float*, int64_t, hipStream_t);
+template hipError_t launch_zero<double>(double*, int64_t, hipStream_t);
 
 }  // namespace pgbsc

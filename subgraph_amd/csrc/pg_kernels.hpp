@@ -215,8 +215,9 @@ hipError_t launch_root_seq(const SubArgs<T>& a, const int4* tiles, int n_tiles, 
 
 // Sums of narrow rows, loaded whole, for tiles of vertices (pg_stream.hip).
 // Tiles {first vertex, vertices, first entry, entries} of up to
-// kStreamTileVertices vertices; local[e]: the place of entry e's vertex in its
-// tile.  n_rows: rows of the gathered table (of less than 4 GB).
+// kStreamTileVertices vertices with an entry each at least; local[e]: the place
+// of entry e's vertex in its tile.  n_rows: rows of the gathered table (of less
+// than 4 GB).
 constexpr int kStreamTileEntries = 256, kStreamTileVertices = 256;
 enum StreamMode : int {
     STREAM_FORWARD = 0,  // GATHER in the reference's order, main a leaf, OUT_EMA or OUT_EMA_SCALED
@@ -324,7 +325,8 @@ hipError_t launch_scatter_grad(TO* out, const double* grad, const double* grad_t
                                const int32_t* ent_tr, int64_t nnz, double factor, hipStream_t st);
 // dst[i] = ids[at[i]]
 hipError_t launch_gather_ids(int32_t* dst, const int32_t* ids, const int32_t* at, int64_t n, hipStream_t st);
-hipError_t launch_zero_f64(double* p, int64_t n, hipStream_t st);
+template <typename T>
+hipError_t launch_zero(T* p, int64_t n, hipStream_t st);
 
 // ---- the reference's unpruned mode (isPruned = 0, CountMat.cpp:851-977) ----
 // One non-leaf subtemplate for one coloring, thread per vertex, exactly the
