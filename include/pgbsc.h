@@ -118,8 +118,9 @@ const char* pg_last_error(const pg_ctx* ctx);
  *                  sweep, 1 rebuilds each table from its subtree when the sweep needs it,
  *                  -1 rebuilds only when that fits four times as many colorings per pass,
  *                  or when kept tables do not fit one coloring (default)
- * Read-only: "last_tile" (colorings per pass of the last count / gradient call) and
- * "last_recompute" (1 if that gradient call rebuilt tables). */
+ * Read-only: "last_tile" (colorings per pass of the last count / gradient call),
+ * "last_recompute" (1 if that gradient call rebuilt tables) and "big_hubs" (hubs whose
+ * neighbour lists, of more than 4096 entries, 16 wavefronts share). */
 int pg_set_option(pg_ctx* ctx, const char* key, int64_t value);
 int pg_get_option(const pg_ctx* ctx, const char* key, int64_t* value);
 

@@ -2938,6 +2938,7 @@ extern "C" int pg_get_option(const pg_ctx* c, const char* key, int64_t* v)
     else if (k == "vertex_order") *v = c->vertex_order;
     else if (k == "last_tile") *v = c->last_tile;
     else if (k == "last_recompute") *v = c->last_recompute;
+    else if (k == "big_hubs") *v = c->n_big;
     else if (k == "graphs") *v = c->use_graphs ? 1 : 0;
     else return PG_ERR_INVALID;
     return PG_OK;
@@ -3018,8 +3019,10 @@ extern "C" int pg_graph_upload(pg_ctx* c, int32_t n, int64_t nnz, const int32_t*
                 }
             }
         }
-        // degree >= bound: hubs above 128, 256, 512, 1024; team buckets from 4 .. 512; a list at all
-        static const int64_t bounds[] = {1025, 513, 512, 257, 256, 129, 128, 64, 32, 16, 8, 4, 1};
+        // degree >= bound: the largest hubs, to which k_hub_seq gives whole workgroups by their prefix
+        // (R-MAT scale 20, 7-vertex tree, one coloring: 1.37 ms where they lie among the hubs above
+        // 1024, 1.21 ms so); hubs above 128, 256, 512, 1024; team buckets from 4 .. 512; a list at all
+        static const int64_t bounds[] = {kHubBigDegree + 1, 1025, 513, 512, 257, 256, 129, 128, 64, 32, 16, 8, 4, 1};
         auto cls = [&](int32_t v) {
             int k = 0;
             for (int64_t b : bounds) {
