@@ -98,6 +98,9 @@ const char* pg_last_error(const pg_ctx* ctx);
  *   "fuse_grad"    pg_count_grad with kept tables: 1 = the forward keeps the Y that the adjoint
  *                  reads, and the transposed gather (by colour runs or per lane) also takes the
  *                  entries' gradients (default); 0 = a gradient gather recomputes Y
+ *                  (FP32 tables: the streamed gathers of narrow rows add up to 64 of an entry's
+ *                  terms, and gradient gathers per lane up to 256, over the pass's colorings
+ *                  in FP32 before its FP64 sum; the others add each coloring's apart)
  *   "fuse_min_width" with fuse_grad: steps whose dY rows have at least this many values, and
  *                  whose per-lane gather has no index table, fuse by colour runs whatever share
  *                  of a row a vertex uses (default 128)

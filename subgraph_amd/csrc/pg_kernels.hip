@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <map>
+#include <type_traits>
 
 namespace pgbsc {
 
@@ -548,14 +549,31 @@ __global__ __launch_bounds__(kBlock) void k_sub(const SubArgs<T> a)
                                     x[q][r] = aux_term<T, AUX>(a, s_rank, amask[r], aoff, uq, cq);
                             }
                         }
+                        if constexpr (AUX == AUX_GATHER_TG && sizeof(T) == 4) {
+                            // four at a time, by pairs: a chain a quarter as long rounds less
+                            // (gradients of the 12-vertex tree, R-MAT scale 14: 9.3e-8 from
+                            // the FP64 ones one by one, 8.5e-8 so; the same time)
 #pragma unroll
-                        for (int q = 0; q < 4; ++q)
+                            for (int r = 0; r < RC; ++r) {
+                                T t[4];
 #pragma unroll
-                            for (int r = 0; r < RC; ++r)
-                                acc[r] = a.w ? acc[r] + wv[q] * x[q][r] : acc[r] + x[q][r];
+                                for (int q = 0; q < 4; ++q) t[q] = a.w ? wv[q] * x[q][r] : x[q][r];
+                                acc[r] = acc[r] + ((t[0] + t[1]) + (t[2] + t[3]));
+                            }
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                                for (int r = 0; r < RC; ++r)
+                                    acc[r] = a.w ? acc[r] + wv[q] * x[q][r] : acc[r] + x[q][r];
+                        }
                         if (edge_grad) {
                             // d Y[v] / d w_e = x_e: contract with dY over the group's
-                            // values in the table precision, one FP64 add per entry.
+                            // values, one FP64 add per entry.  A lane's RC values are
+                            // of one coloring; the lanes' sums span the colorings of the
+                            // pass, whose cotangents may cancel, and are FP64 where the
+                            // launch stands for whole-row gathers that add each
+                            // coloring to the entry in FP64 (TG).
                             // The 4 neighbours' dots reduce together (fixed order):
                             // xor 1 and xor 2 halve the values a lane carries, so lane
                             // bits (0,1) end up naming the neighbour 2*b0 + b1, then
@@ -572,18 +590,19 @@ __global__ __launch_bounds__(kBlock) void k_sub(const SubArgs<T> a)
 #pragma unroll
                                 for (int r = 0; r < RC; ++r) dot[q] = dot[q] + dyv[r] * x[q][r];
                             }
+                            using S = std::conditional_t<AUX == AUX_GATHER_TG, double, T>;
                             if (cl >= 4) {
                                 const bool h1 = cln & 1, h2 = (cln >> 1) & 1;
-                                const T pa = (h1 ? dot[2] : dot[0]) + __shfl_xor(h1 ? dot[0] : dot[2], 1, TEAM);
-                                const T pb = (h1 ? dot[3] : dot[1]) + __shfl_xor(h1 ? dot[1] : dot[3], 1, TEAM);
-                                T sum = (h2 ? pb : pa) + __shfl_xor(h2 ? pa : pb, 2, TEAM);
+                                const S pa = (S)(h1 ? dot[2] : dot[0]) + (S)__shfl_xor(h1 ? dot[0] : dot[2], 1, TEAM);
+                                const S pb = (S)(h1 ? dot[3] : dot[1]) + (S)__shfl_xor(h1 ? dot[1] : dot[3], 1, TEAM);
+                                S sum = (h2 ? pb : pa) + __shfl_xor(h2 ? pa : pb, 2, TEAM);
                                 for (int sh = 4; sh < cl; sh <<= 1) sum = sum + __shfl_xor(sum, sh, TEAM);
                                 const int q = 2 * (int)h1 + (int)h2;
                                 if (cln < 4 && ok[q]) (void)unsafeAtomicAdd(&a.grad[e + q * step], (double)sum);
                             } else {
 #pragma unroll
                                 for (int q = 0; q < 4; ++q) {
-                                    T sum = dot[q];
+                                    S sum = dot[q];
                                     for (int sh = 1; sh < cl; sh <<= 1) sum = sum + __shfl_xor(sum, sh, TEAM);
                                     if (cln == 0 && ok[q]) (void)unsafeAtomicAdd(&a.grad[e + q * step], (double)sum);
                                 }

@@ -128,10 +128,11 @@ __device__ __forceinline__ float lane_sums(const float (&p)[16], int lane)
 
 // TG: the adjoint's transposed gather, which also takes the gradient of each
 // entry's transpose, the dot of what the entry adds with the vertex's own row:
-// grad[e] += sum over lanes of dy[v] * x, for 16 entries at a time by adds that
-// leave each entry's sum in four lanes (lane_sums; a reduction of its own per
-// entry would take six).  HUB: tiles are {vertex, first entry, end entry,
-// output row}, parts of one list each.
+// grad[e] += sum over lanes of dy[v] * x, in FP32 over the wavefront's colorings
+// (up to 64 values; the gradient gather adds up to 256), for 16 entries at a
+// time by adds that leave each entry's sum in four lanes (lane_sums; a reduction
+// of its own per entry would take six).  HUB: tiles are {vertex, first entry,
+// end entry, output row}, parts of one list each.
 template <typename T, int NB, bool TG, bool HUB>
 __global__ __launch_bounds__(kBlock) void k_stream(const SubArgs<T> a, const int4* tiles, int n_tiles,
                                                    const uint8_t* local, int CB, int nch, uint32_t table_bytes)
