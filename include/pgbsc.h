@@ -96,7 +96,7 @@ const char* pg_last_error(const pg_ctx* ctx);
  *   "color_runs"   whole-row neighbour sums: 1 always (rows up to 512 values), 0 never,
  *                  -1 by row width and used share (default)
  *   "fuse_grad"    pg_count_grad with kept tables: 1 = the forward keeps the Y that the adjoint
- *                  reads, and the transposed gather (by colour runs or per lane) also takes the
+ *                  reads, as far as the memory allows, and the transposed gather (by colour runs or per lane) also takes the
  *                  entries' gradients (default); 0 = a gradient gather recomputes Y
  *                  (FP32 tables: the streamed gathers of narrow rows add up to 64 of an entry's
  *                  terms, and gradient gathers per lane up to 256, over the pass's colorings

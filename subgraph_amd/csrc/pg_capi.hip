@@ -74,7 +74,7 @@ struct GraphKey {
     const void* colors_in;  // caller colors buffer, nullptr = device RNG
     const void* arena;
     uint64_t generation;    // graph / weights / bucket version
-    int kind = 0;           // 0 count pass, 1 gradient pass (kept tables), 2 gradient pass (rebuilt tables)
+    int kind = 0;           // 0 count pass, 1 gradient pass (rebuilt tables), 2 + KeepY gradient pass (kept tables)
     const void* grad = nullptr;  // gradient accumulator of a gradient pass
     bool operator<(const GraphKey& o) const
     {
@@ -1910,9 +1910,19 @@ int build_transpose(pg_ctx* c)
 // keep_all every forward table and every G_s has its own slot for the whole
 // pass; otherwise (recompute) the tables live in a pool above the pass-long
 // buffers, and off_pool / pool_bytes describe it.
+// The steps whose Y the forward pass keeps beside the tables: a step whose
+// node launch would read it and that has none takes a gather of its own for
+// the entries' gradients, which makes Y again.
+enum KeepY : int {
+    KEEP_Y_NONE = 0,
+    KEEP_Y_ROWS = 1,  // of whole-row gathers (fused_grad_step)
+    KEEP_Y_ALL = 2,   // and of per-lane ones (lane_grad_step)
+};
+
 struct GradPlan {
     MemPlan fwd;
     bool keep_all = true;
+    KeepY keep_y = KEEP_Y_NONE;
     std::vector<size_t> off_G;
     size_t off_Y = 0, off_dY = 0, off_cot = 0, off_pool = 0, pool_bytes = 0, total = 0;
 };
@@ -1973,9 +1983,10 @@ SubArgs<T> transposed_args(const pg_ctx* c, const DevSub& d, int B, SubArgs<T> t
     return t;
 }
 
-GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
+GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz, KeepY keep_y)
 {
     GradPlan g;
+    g.keep_y = keep_y;
     g.fwd = plan_memory(c, p, B, tsz);
     // forward plan reuses table space; give every table its own slot instead
     size_t off = g.fwd.total;
@@ -1994,7 +2005,9 @@ GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
     for (auto& d : p->subs) {
         // Y kept for the steps without a gradient gather (which recomputes
         // it), where the node launch reads it
-        if (!fused_grad_step(c, p, *d) && !(lane_grad_step(c, p, *d) && d->mm > 1)) continue;
+        const bool keeps = (keep_y >= KEEP_Y_ROWS && fused_grad_step(c, p, *d)) ||
+                           (keep_y >= KEEP_Y_ALL && d->mm > 1 && lane_grad_step(c, p, *d));
+        if (!keeps) continue;
         g.fwd.off_ykeep[d->s] = off;
         off += align_up((size_t)c->n_act * B * d->Wy * tsz, 256);
     }
@@ -2008,6 +2021,16 @@ GradPlan plan_memory_grad(const pg_ctx* c, const pg_plan* p, int B, size_t tsz)
     off += align_up((size_t)B * sizeof(double), 256);
     g.total = off;
     return g;
+}
+
+// Y of step s as plan g keeps it for the adjoint (0: not kept)
+size_t kept_y(const GradPlan& g, int s) { return (size_t)s < g.fwd.off_ykeep.size() ? g.fwd.off_ykeep[s] : 0; }
+
+// Whether the transposed gather of step d takes its entries' gradients per
+// lane (lane_grad_step): with Y kept, or where the node launch needs none.
+bool by_lane_step(const pg_ctx* c, const pg_plan* p, const DevSub& d, bool y_kept)
+{
+    return (y_kept || d.mm == 1) && lane_grad_step(c, p, d);
 }
 
 // The dY of steps with a leaf aux child whose entries' gradients wait for a
@@ -2102,7 +2125,7 @@ int enqueue_sub_backward(pg_ctx* c, const pg_plan* p, const DevSub& d, int B, co
     // per-entry gradient read and written by each launch that adds to it.
     const double col = 4.0 * (double)c->n_act * B, Z = (double)c->nnz;
     const double Cs = d.root ? 0.0 : d.Cs, Cm = d.mm > 1 ? d.Cm : 0.0, Ca = d.Ca;
-    const bool by_lane = lane_grad_step(c, p, d) && (Yk || d.mm == 1);
+    const bool by_lane = by_lane_step(c, p, d, Yk != nullptr);
     if (d.aa > 1 && (Yk || by_lane)) {
         // dY and G_main from G, the main row and the kept Y
         na.Y = Yk;
@@ -2207,7 +2230,7 @@ int enqueue_backward_kept(pg_ctx* c, const pg_plan* p, int B, const GradPlan& gp
     bool waits_in_dYbuf = false;
     for (auto it = p->subs.rbegin(); it != p->subs.rend(); ++it) {
         const DevSub& d = **it;
-        const size_t yk = (size_t)d.s < gp.fwd.off_ykeep.size() ? gp.fwd.off_ykeep[d.s] : 0;
+        const size_t yk = kept_y(gp, d.s);
         // A leaf aux child's dY waits for the common launch in the step's own
         // forward table, which only the steps above it, done by now, read; the
         // root, which has none, uses the common buffer.
@@ -2398,17 +2421,34 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         for (auto& d : p->subs) lds = std::max(lds, sub_lds_max(c, p, *d, B, tsz));
         return lds <= kLdsLimit;
     };
-    int tile_keep = 0, tile_rec = 0;
-    GradPlan g_keep, g_rec;
+    // Kept tables with all the Y that fused gradient gathers need (KeepY), or
+    // with less of it where that leaves no room for one coloring or, for narrow
+    // templates, the per-lane steps' halves a pass.  R-MAT scale 18 (20 for 12
+    // vertices), FP32, ms a coloring, one per pass with those steps' Y / two
+    // without: 7 vertices 1.59 / 1.11, 10 vertices 5.71 / 5.89, 12 vertices
+    // 38.7 / 46.3; two / four: 0.96 / 0.84, 12 vertices 37.2 / 44.3.  At the
+    // same number the Y gains 13-24%.
+    constexpr int kNarrowTemplate = 9;
+    int tile_of_keep[3] = {0, 0, 0}, tile_rec = 0;  // the widest passes that fit, by KeepY
+    GradPlan g_of_keep[3], g_rec;
+    auto kept = [&](int B, KeepY y) { return plan_memory_grad(c, p, B, tsz, y); };
     if (c->adjoint_recompute != 1)
-        for (int B = cap; B >= 1; --B) {
+        for (int B = cap, y = KEEP_Y_NONE; B >= 1 && y <= KEEP_Y_ALL; --B) {
             if (!lds_ok(B)) continue;
-            GradPlan g = plan_memory_grad(c, p, B, tsz);
-            if (g.total > budget) continue;
-            tile_keep = B;
-            g_keep = g;
-            break;
+            // more Y needs more memory: where all of it fits, so does less
+            const GradPlan all = kept(B, KEEP_Y_ALL);
+            const bool fits = all.total <= budget;
+            for (; y <= KEEP_Y_ALL; ++y) {
+                g_of_keep[y] = fits || y == KEEP_Y_ALL ? all : kept(B, (KeepY)y);
+                if (g_of_keep[y].total > budget) break;
+                tile_of_keep[y] = B;
+            }
         }
+    const int t_rows = tile_of_keep[KEEP_Y_ROWS], t_all = tile_of_keep[KEEP_Y_ALL];
+    const KeepY keep_y = t_all > 0 && (p->k > kNarrowTemplate || t_rows < 2 * t_all) ? KEEP_Y_ALL
+                         : t_rows > 0                                                ? KEEP_Y_ROWS
+                                                                                     : KEEP_Y_NONE;
+    const int tile_keep = t_rows > 0 ? t_rows : tile_of_keep[KEEP_Y_NONE];
     const int rec_lo = c->adjoint_recompute == 1 ? 1 : tile_keep == 0 ? 1 : tile_keep * kRecomputeGain;
     if (c->adjoint_recompute != 0)
         for (int B = cap; B >= rec_lo; --B) {
@@ -2420,8 +2460,8 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
             break;
         }
     const bool use_rec = tile_rec > 0;
-    int tile = use_rec ? tile_rec : tile_keep;
-    GradPlan gp = use_rec ? g_rec : g_keep;
+    int tile = use_rec ? tile_rec : tile_of_keep[keep_y];
+    GradPlan gp = use_rec ? g_rec : g_of_keep[keep_y];
     if (tile == 0) return set_err(c, PG_ERR_NOMEM, "adjoint tables of one coloring do not fit the device");
     c->last_tile = tile;
     c->last_recompute = use_rec ? 1 : 0;
@@ -2444,7 +2484,12 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
         if (rt) return rt;
         if (fwd_tile >= 1 && fwd_tile < tile) tile = fwd_tile;
         c->last_tile = tile;
-        gp = use_rec ? plan_memory_recompute<T>(c, p, tile, budget) : plan_memory_grad(c, p, tile, tsz);
+        if (use_rec) gp = plan_memory_recompute<T>(c, p, tile, budget);
+        else
+            for (int y = KEEP_Y_ALL; y >= keep_y; --y) {  // (a smaller tile may hold more of the Y)
+                gp = kept(tile, (KeepY)y);
+                if (gp.total <= budget) break;
+            }
     }
     if (gp.total > c->d_arena.bytes) {
         drop_graphs(c);
@@ -2462,7 +2507,10 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
     // the entries' gradients and, where a transposed gather takes them in list
     // order (AUX_GATHER_TG, RUNS_TG), those of their transposes
     bool by_transpose = false;
-    for (auto& d : p->subs) by_transpose |= lane_grad_step(c, p, *d) || fused_grad_step(c, p, *d);
+    for (auto& d : p->subs) {
+        const bool y = kept_y(gp, d->s) != 0;
+        by_transpose |= by_lane_step(c, p, *d, y) || (y && fused_grad_step(c, p, *d));
+    }
     const int64_t n_acc = c->nnz * (by_transpose ? 2 : 1);
     HIP_TRY(c, c->d_grad.alloc(std::max<int64_t>(n_acc, 1) * 8));
     HIP_TRY(c, launch_zero<double>(c->d_grad.as<double>(), n_acc, c->stream));
@@ -2487,7 +2535,7 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
     for (int first = 0; first < ncol && rc == PG_OK; first += tile) {
         const int B = std::min(tile, ncol - first);
         const GradPlan g = B == tile ? gp : use_rec ? plan_memory_recompute<T>(c, p, B, gp.total)
-                                                    : plan_memory_grad(c, p, B, tsz);
+                                                    : kept(B, gp.keep_y);
         if (g.total > gp.total) {
             rc = set_err(c, PG_ERR_NOMEM, "adjoint plan of the last pass exceeds the first");
             break;
@@ -2525,7 +2573,7 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
             c->cur_recs = nullptr;
         } else {
             GraphKey key{p, B, (int)tsz, d_in, c->d_arena.p, c->generation};
-            key.kind = use_rec ? 2 : 1;
+            key.kind = use_rec ? 1 : 2 + gp.keep_y;
             key.grad = c->d_grad.p;
             auto it = c->graphs.find(key);
             if (it == c->graphs.end()) {
