@@ -67,7 +67,8 @@ const char* pg_last_error(const pg_ctx* ctx);
  *   "bucket_high"  vertices of at least this degree get 64-lane teams (default 512)
  *   "bucket_mid"   ... at least this degree 16-lane teams, the rest 8 (default 64)
  *   "batch_tile"   colorings per pass, 0 = automatic (default 0)
- *   "mem_budget_mb" device bytes the tables may use, 0 = 90% of free memory
+ *   "mem_budget_mb" device bytes the tables may use, 0 = 90% of free memory (gradient calls:
+ *                  80% of what their per-entry buffers leave)
  *   "autotune"     1 = before the first pass of each (plan, batch tile, precision), time
  *                  one pass per candidate of reg_cols, stage_rows, aux_rows, bucket_high,
  *                  bucket_mid, hub_degree and hub_chunk and keep
@@ -96,8 +97,9 @@ const char* pg_last_error(const pg_ctx* ctx);
  *   "color_runs"   whole-row neighbour sums: 1 always (rows up to 512 values), 0 never,
  *                  -1 by row width and used share (default)
  *   "fuse_grad"    pg_count_grad with kept tables: 1 = the forward keeps the Y that the adjoint
- *                  reads, as far as the memory allows, and the transposed gather (by colour runs or per lane) also takes the
- *                  entries' gradients (default); 0 = a gradient gather recomputes Y
+ *                  reads, as far as the memory allows, and the transposed gather (by colour
+ *                  runs or per lane) also takes the entries' gradients (default); 0 = a
+ *                  gradient gather recomputes Y
  *                  (FP32 tables: the streamed gathers of narrow rows add up to 64 of an entry's
  *                  terms, and gradient gathers per lane up to 256, over the pass's colorings
  *                  in FP32 before its FP64 sum; the others add each coloring's apart)

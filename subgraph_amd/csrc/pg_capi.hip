@@ -2405,7 +2405,17 @@ int count_grad_impl(pg_ctx* c, const pg_plan* p, int ncol, const uint8_t* colors
     } else {
         size_t fr = 0, tot = 0;
         HIP_TRY(c, hipMemGetInfo(&fr, &tot));
-        budget = (size_t)(0.8 * (double)(fr + c->d_arena.bytes));
+        // beside the tables: the entries' gradients and their transposes', the
+        // transposed weights, the caller's colors and the host copy of the
+        // result, as far as no earlier call made them
+        auto grows = [](const DevBuf& b, size_t need) { return need > b.bytes ? need - b.bytes : 0; };
+        const size_t nnz = (size_t)c->nnz;
+        size_t beside = grows(c->d_grad, 2 * nnz * sizeof(double));
+        if (c->weighted) beside += grows(tsz == 4 ? c->d_wT32 : c->d_wT64, nnz * tsz);
+        if (colors) beside += grows(c->d_colors_in, (size_t)ncol * c->n);
+        if (grad && !grad_on_device) beside += grows(c->d_grad_out, nnz * sizeof(double));
+        const size_t free_bytes = fr + c->d_arena.bytes;
+        budget = (size_t)(0.8 * (double)(free_bytes > beside ? free_bytes - beside : 0));
     }
     // the largest batch tile that fits, with every table kept and with tables
     // recomputed; option "adjoint_recompute": 0 keep, 1 recompute, -1 keep

@@ -57,3 +57,39 @@ def test_tables_that_just_fit_are_enough(gpu_ctx, k, edges, scale, precision):
     finally:
         for key, v in zip(KEYS, saved):
             gpu_ctx.set_option(key, v)
+
+
+@pytest.mark.gpu
+def test_entry_buffers_are_left_room(gpu_ctx):
+    """With little memory free, the tables of a gradient call leave room for its
+    buffers per entry (some 28 bytes each beside the tables, of 1.3 GB free for
+    18 million entries): the call runs, and gives what it gives with memory to
+    spare, to FP32 rounding (1e-5, gradients in norm; a weighted histogram's order
+    depends on the colorings of a pass)."""
+    torch = pytest.importorskip("torch")
+    n, mb = 150_000, 1 << 20
+    rng = np.random.default_rng(103)
+    a, b = rng.integers(0, n, 9_000_000), rng.integers(0, n, 9_000_000)
+    key = np.unique(np.minimum(a, b)[a != b] * n + np.maximum(a, b)[a != b])
+    colptr, rowidx = sg.csc_from_edges(n, (key // n).astype(np.int32), (key % n).astype(np.int32))
+    ctx = sg.Context(0)
+    ctx.upload_graph(colptr, rowidx)
+    ctx.set_weights(rng.uniform(0.5, 1.5, len(rowidx)).astype(np.float32))
+    plan = ctx.plan(7, TREE7)
+    hold = []
+    try:
+        ctx.count(plan, 1, seed=9, precision="fp32")
+        for keep, piece in ((4096, 2048), (1500, 128)):  # MB free, MB at a time
+            while torch.cuda.mem_get_info()[0] > (keep + piece) * mb:
+                hold.append(torch.empty(piece * mb, dtype=torch.uint8, device="cuda"))
+        print(f"[tight memory] {torch.cuda.mem_get_info()[0] // mb} MB free, {len(rowidx)} entries", flush=True)
+        raw, grad = ctx.count_grad(plan, 64, seed=9, precision="fp32")
+        print(f"[tight memory] {ctx.get_option('last_tile')} colorings a pass", flush=True)
+        assert 1 <= ctx.get_option("last_tile") < 64 and ctx.get_option("last_recompute") == 0
+    finally:
+        hold.clear()
+        torch.cuda.empty_cache()
+    ample, want = ctx.count_grad(plan, 64, seed=9, precision="fp32")
+    assert ctx.get_option("last_tile") == 64
+    assert np.allclose(raw, ample, rtol=1e-5, atol=0)
+    assert np.linalg.norm(grad - want) <= 1e-5 * np.linalg.norm(want)
