@@ -3498,12 +3498,13 @@ extern "C" int pg_plan_footprint(pg_ctx* c, const pg_plan* p, int B, int precisi
     if (device_bytes) {
         size_t b = plan_memory(c, p, B, tsz).total;
         const DevBuf* graph_bufs[] = {&c->d_rowptr, &c->d_col, &c->d_ent, &c->d_perm, &c->d_w32, &c->d_w64,
-                                      &c->d_wsrc, &c->d_hub_items, &c->d_slot_begin, &p->rank_tab};
+                                      &c->d_wsrc, &c->d_hub_items, &c->d_slot_begin, &c->d_hub_iota,
+                                      &c->d_root_tiles, &c->d_stream_tiles, &c->d_local, &p->rank_tab};
         for (const DevBuf* g : graph_bufs)
             b += g->bytes;
         for (auto& d : p->subs)
             for (const DevBuf* t : {&d->split, &d->ymask, &d->by_aux, &d->by_main, &d->by_auxT, &d->by_mainT,
-                                    &d->amask, &d->gidx, &d->xidx, &d->gidxT})
+                                    &d->amask, &d->gidx, &d->xidx, &d->xidx_g, &d->gidxT, &d->ttab})
                 b += t->bytes;
         *device_bytes = (int64_t)b;
     }
