@@ -911,10 +911,7 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         }
         return PG_OK;
     };
-    // (a histogram over few entries takes less than the fork and join: 3-path,
-    // one coloring, scale 16, 1.8 million entries 0.151 ms without, 0.160 with;
-    // scale 18, 7.6 million 0.257 either way; 16 colorings of the 5-path, scale
-    // 16, 29 million 0.54 without, 0.50 with)
+    // (a histogram over few entries takes less than the fork and join)
     const bool fork = aux != AUX_COLORS || (double)c->nnz * a.B > (1 << 22);
     const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest, fork);
     if (frc) return frc;
@@ -1083,12 +1080,17 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         }
         return gather(a, c->n_hub, c->n_act, main_mode, stream, rs);
     };
-    // Side by side (one after the other): 5-path, R-MAT scale 16, one coloring
-    // 0.30 ms (0.36); 10-vertex tree, scale 18, 4 colorings 7.1 (8.1); 12-vertex,
-    // scale 20, 4 colorings 65.5 (70.7); the same within 1% for the 3-path at
-    // scale 16 (0.152, 0.151) and for 64 colorings of the 7-vertex tree (scale 20:
-    // 35.2 either way), 9% more for those of the 3-path there (4.04, 3.69).
-    const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest);
+    // Side by side unless that gains nothing: where the longest list's chain
+    // (4.4 ns an entry) is less than a twentieth of the hub launch's work (0.037
+    // ns per entry and wavefront unit), the two launches only compete (7-vertex
+    // tree, R-MAT scale 20, 64 colorings: 42.1 ms side by side, 39.2 ms one after
+    // the other); and where the other launch is a root's over few entries, a
+    // fork and join cost more than it takes (3-path, scale 16: 162 against 152
+    // us).
+    const double hub_work = 0.037 * c->h_rowptr[c->n_hub] * ((a.B * (double)a.Wy + 63) / 64);
+    const double rest_entries = ((double)c->nnz - c->h_rowptr[c->n_hub]) * a.B;
+    const bool fork = (a.Wy > 48 || 4.4 * c->max_deg > 0.05 * hub_work) && (!root_tiles || rest_entries > (1 << 21));
+    const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest, fork);
     if (frc) return frc;
     if (c->n_hub > 0) {
         SubArgs<T> f = a;
