@@ -911,7 +911,10 @@ int launch_gathering(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* part, i
         }
         return PG_OK;
     };
-    // (a histogram over few entries takes less than the fork and join)
+    // (a histogram over few entries takes less than the fork and join: 3-path,
+    // one coloring, scale 16, 1.8 million entries 0.151 ms without, 0.160 with;
+    // scale 18, 7.6 million 0.257 either way; 16 colorings of the 5-path, scale
+    // 16, 29 million 0.54 without, 0.50 with)
     const bool fork = aux != AUX_COLORS || (double)c->nnz * a.B > (1 << 22);
     const int frc = fork_hubs(c, c->n_hub > 0, hubs, rest, fork);
     if (frc) return frc;
@@ -1080,13 +1083,16 @@ int launch_gathering_exact(pg_ctx* c, int aux, int main_mode, SubArgs<T> a, T* p
         }
         return gather(a, c->n_hub, c->n_act, main_mode, stream, rs);
     };
-    // Side by side unless that gains nothing: where the longest list's chain
-    // (4.4 ns an entry) is less than a twentieth of the hub launch's work (0.037
-    // ns per entry and wavefront unit), the two launches only compete (7-vertex
-    // tree, R-MAT scale 20, 64 colorings: 42.1 ms side by side, 39.2 ms one after
-    // the other); and where the other launch is a root's over few entries, a
-    // fork and join cost more than it takes (3-path, scale 16: 162 against 152
-    // us).
+    // Side by side unless that gains nothing.  Where the longest list's chain (4.4
+    // ns an entry) is less than a twentieth of the hub launch's work (0.037 ns per
+    // entry and wavefront unit), the two launches only compete: 7-vertex tree, 64
+    // colorings, R-MAT scale 22, hubs above 4,096, a call 323 ms side by side, 282
+    // with the rule; scale 20, hubs above 512, 35.2 either way.  Rows of more than
+    // 48 values, a wavefront unit a coloring, gain all the same: 10-vertex tree, 4
+    // colorings, scale 22, 123 ms side by side, 136 by the rule alone; 12-vertex
+    // tree, scale 20, 65.5 and 66.2.  Where the other launch is a root's over few
+    // entries both measure about the same (scale 16, one coloring: 3-path 152 us
+    // side by side, 150 one after the other; 5-path 299 and 303).
     const double hub_work = 0.037 * c->h_rowptr[c->n_hub] * ((a.B * (double)a.Wy + 63) / 64);
     const double rest_entries = ((double)c->nnz - c->h_rowptr[c->n_hub]) * a.B;
     const bool fork = (a.Wy > 48 || 4.4 * c->max_deg > 0.05 * hub_work) && (!root_tiles || rest_entries > (1 << 21));

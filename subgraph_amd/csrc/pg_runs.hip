@@ -574,7 +574,7 @@ void k_runs_tg(const SubArgs<T> a)
     const int Wg = a.Wa;  // values per colouring of a neighbour's dY row
     const int Wt = a.Wy;  // values per colouring of the G_aux row (and of the own row)
     unsigned char* tb = smem_raw + (size_t)team * runs_tg_team_bytes<T>(Wt);
-    int4* sQ = reinterpret_cast<int4*>(tb);  // (neighbour, transposed entry, colour, -)
+    int4* sQ = reinterpret_cast<int4*>(tb);  // (neighbour, entry, colour, -)
     T* sW = reinterpret_cast<T*>(tb + 16 * TEAM);
     T* sY = sW + TEAM;
     T* sO = sY + Wt;
