@@ -731,10 +731,10 @@ def record_name(symbol):
         s = s.replace(junk, "")
     m = re.match(r"(k_\w+)<(.*)>$", s)
     if not m:
-        return {"k_combine_rows": "k_combine_rows<float>", "k_edge_colors_word": "k_edge_colors"}.get(s, s)
+        return {"k_combine_rows": "k_combine_rows<float>"}.get(s, s)
     name, a = m.group(1), m.group(2).split(",")
-    if name == "k_edge_colors":
-        return name
+    if name in ("k_edge_colors", "k_edge_colors_word"):
+        return "k_edge_colors"
     if name == "k_sub" and len(a) == 5:
         return "k_sub<" + ",".join(a[:4] + ([] if a[4] == "4" else ["1"])) + ">"
     if name in ("k_hub_seq", "k_root_seq"):
